@@ -19,8 +19,8 @@ namespace {
 // outward by half a step keeps a margin far above the slab test's rounding error at any
 // coordinate in the scene. Lower planes round down to floor(x - 1/2) (clamped at the node's
 // origin, which is a child's own padded bound), upper planes up to ceil(x + 1/2) <= 255.
-// Returns false (no quantised layout) when an exponent leaves [-100, 60], where 2^e times an
-// inverse direction could leave the normal float range.
+// Returns false (no quantised layout) when an exponent leaves [-100, 36], where 2^(e + 24) times
+// an inverse direction (at most 1e20) could leave the float range.
 bool quantize4(const std::vector<GpuNode4>& in, std::vector<GpuNodeQ>& out)
 {
     out.assign(in.size(), GpuNodeQ{});
@@ -44,11 +44,12 @@ bool quantize4(const std::vector<GpuNode4>& in, std::vector<GpuNodeQ>& out)
         uint32_t* qhi[3] = {&q.qhix, &q.qhiy, &q.qhiz};
         q.exps = 0;
         q.cnts = 0;
-        q.pad = 0;
+        q.leaf_bits = 0;
         for (int c = 0; c < 4; ++c)
         {
             q.ref[c] = g.ref[c];
             q.cnts |= (uint32_t)(uint8_t)(int8_t)g.cnt[c] << (8 * c);
+            if (g.cnt[c] > 0) q.leaf_bits |= ((1u << g.cnt[c]) - 1u) << (8 * c);
         }
         for (int a = 0; a < 3; ++a)
         {
@@ -64,7 +65,7 @@ bool quantize4(const std::vector<GpuNode4>& in, std::vector<GpuNodeQ>& out)
             int e;
             std::frexp(std::max(ext / 254.0, floor_step), &e);   // 2^(e-1) <= x < 2^e
             if (std::ldexp(1.0, e - 1) >= std::max(ext / 254.0, floor_step)) --e;
-            if (e < -100 || e > 60) return false;
+            if (e < -100 || e > 36) return false;
             const double step = std::ldexp(1.0, e);
             q.origin[a] = o;
             q.exps |= (uint32_t)(uint8_t)(int8_t)e << (8 * a);
@@ -145,7 +146,7 @@ public:
     Builder(const float* tv, size_t n, const BuildParams& p) : tv_(tv), n_(n), p_(p)
     {
         if (p_.max_leaf < 1) p_.max_leaf = 1;
-        if (p_.max_leaf > 8) p_.max_leaf = 8;
+        if (p_.max_leaf > kMaxLeaf) p_.max_leaf = kMaxLeaf;
         if (p_.bins < 4) p_.bins = 4;
         if (p_.bins > 64) p_.bins = 64;
         threads_ = p_.threads > 0 ? p_.threads : (int)std::max(1u, std::thread::hardware_concurrency());
@@ -395,14 +396,17 @@ private:
     void flatten4(int root, BuildOutput& out)
     {
         out.nodes4.clear();
-        out.tri_order.assign(idx_.begin(), idx_.end());
+        out.tri_order.clear();
+        out.tri_order.reserve(n_);
         out.max_depth = 0;
         out.nodes4.reserve(ncount_.load() / 2 + 1);
         emit4(root, 0, out);
     }
 
     // Children of a 4-wide node: start from the BVH2 node's two children and open the
-    // internal one of largest area until there are four or only leaves remain.
+    // internal one of largest area until there are four or only leaves remain. Leaf children
+    // take the first slots, and their triangles are numbered consecutively before any
+    // descendant's, so triangle j of the node's leaves is ref[0] + j.
     int emit4(int t, int depth, BuildOutput& out)
     {
         out.max_depth = std::max(out.max_depth, depth);
@@ -425,6 +429,7 @@ private:
             kids[best] = nodes_[open].left;
             kids[nk++] = nodes_[open].right;
         }
+        std::stable_partition(kids, kids + nk, [&](int k) { return nodes_[k].left < 0; });
         ChildRef c[4];
         for (int k = 0; k < 4; ++k)
         {
@@ -439,8 +444,10 @@ private:
             c[k].box = ch.box;
             if (ch.left < 0)
             {
-                c[k].ref = ch.first;
+                c[k].ref = (int)out.tri_order.size();
                 c[k].count = ch.count;
+                out.tri_order.insert(out.tri_order.end(), idx_.begin() + ch.first,
+                                     idx_.begin() + ch.first + ch.count);
             }
             else
             {

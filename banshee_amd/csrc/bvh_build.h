@@ -30,7 +30,8 @@ static_assert(sizeof(GpuNode) == 64, "node is 64 B");
 
 // 4-wide node, 128 B = 8 x float4: per child slab bounds, then refs and counts (same
 // meaning as in GpuNode). Collapsed from the binned-SAH BVH2 by repeatedly opening the
-// internal child of largest surface area, so one visit tests up to four boxes.
+// internal child of largest surface area, so one visit tests up to four boxes. Leaf children
+// come first, and the triangles of a node's leaves are consecutive from ref[0] on.
 struct GpuNode4
 {
     float lox[4], hix[4], loy[4], hiy[4], loz[4], hiz[4];
@@ -44,20 +45,21 @@ static_assert(sizeof(GpuNode4) == 128, "node is 128 B");
 // "Efficient incoherent ray traversal on GPUs through compressed wide BVHs", HPG 2017):
 //   w0 = (origin.x, origin.y, origin.z, exponents as signed bytes: e_x | e_y << 8 | e_z << 16)
 //   w1 = (qlo.x, qhi.x, qlo.y, qhi.y), each 4 bytes, byte c for child c
-//   w2 = (qlo.z, qhi.z, counts as 4 signed bytes, 0)
+//   w2 = (qlo.z, qhi.z, counts as 4 signed bytes, leaf bits: byte c holds one low bit per
+//        triangle of leaf child c, 0 for other children)
 //   w3 = refs (as in GpuNode4)
 // Child c's box on axis a is [origin + qlo 2^e, origin + qhi 2^e]. The builder rounds every plane
 // outward by at least half a grid step (a lower plane of 0 is the node's own padded bound), and
 // the grid step is at least 2^-17 of the scene's largest coordinate, so the traversal's rounding
 // of these planes stays inside the margin and the boxes contain the float boxes they replace.
-// e stays within [-100, 60].
+// e stays within [-100, 36].
 struct GpuNodeQ
 {
     float origin[3];
     uint32_t exps;
     uint32_t qlox, qhix, qloy, qhiy, qloz, qhiz;
     uint32_t cnts;
-    uint32_t pad;
+    uint32_t leaf_bits;
     int32_t ref[4];
 };
 static_assert(sizeof(GpuNodeQ) == 64, "node is 64 B");
@@ -69,6 +71,9 @@ constexpr int kMaxStack = 32;
 // The 4-wide traversal pushes at most 3 children per level; the builder falls back to the
 // binary layout when 3 x (4-wide depth) + 1 would exceed this.
 constexpr int kMaxStack4 = 48;
+// Largest triangle count of a leaf (bsh_bvh_params.max_leaf is clamped to it): the traversal
+// marks a node's hit triangles in 8 bits per child.
+constexpr int kMaxLeaf = 8;
 
 struct BuildParams
 {

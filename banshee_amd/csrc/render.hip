@@ -42,6 +42,7 @@
 #include "shading.h"
 #include "sh_dev.h"
 #include "guide_dev.h"
+#include "trace_core.h"
 
 namespace bsh {
 
@@ -451,73 +452,37 @@ __global__ __launch_bounds__(kBlock) void k_trace_queue(RenderDev R, int L, int 
     }
 }
 
-// The trace stack with its top entry in a register: entries 0 .. sp-2 in LDS (past kTraceLds in
-// the global overflow), entry sp-1 in `top`. A pop returns the register at once and refills it
-// from LDS, so the next node's fetch does not wait for an LDS read.
-__device__ __forceinline__ void push_top(lu32* stk, gu32* ovf, int ostride, int& sp, uint32_t& top, uint32_t v)
+// The overflow slots of a trace thread's stack: entries past kTraceLds, [entry][trace thread].
+struct QueueOvf
 {
-    if (sp >= kMaxStack4) return;   // the builder bounds the depth, so this never drops an entry
-    if (sp > 0)
-    {
-        const int p = sp - 1;
-        if (p < kTraceLds) stk[p * kBlock] = top;
-        else ovf[(p - kTraceLds) * ostride] = top;
-    }
-    top = v;
-    ++sp;
-}
+    gu32* p;
+    int stride;
+    __device__ __forceinline__ gu32& at(int i) const { return p[(size_t)i * stride]; }
+};
 
-__device__ __forceinline__ uint32_t pop_top(lu32* stk, gu32* ovf, int ostride, int& sp, uint32_t& top)
-{
-    const uint32_t v = top;
-    --sp;
-    if (sp > 0)
-    {
-        const int p = sp - 1;
-        top = p < kTraceLds ? stk[p * kBlock] : ovf[(p - kTraceLds) * ostride];
-    }
-    return v;
-}
-
-// 4-wide traversal with per-lane refill. The closest-hit queue and the any-hit queue form one
-// index range [0, nc + na) drawn by one work counter. Every lane holds its own ray state and
-// advances it by one step per loop iteration (a leaf triangle, the sort of a visit's children
-// and the next visit, as far as each applies); a finished lane idles until `refill` or
-// more lanes of its wave are idle (or the whole wave is), when the wave claims exactly that
-// many new rays with one atomic and hands them to the idle lanes in lane order. Lanes of one
-// wave may hold closest and any-hit rays of different scenes at once. Node visits and
-// accept rules are those of traverse4, so every ray's result is the same. kQ: every scene of
-// the launch has GpuNodeQ nodes (else every one has GpuNode4 nodes). kOne: every job traces
-// one scene (R.nodes1), whose arrays then stay in scalar registers.
+// 4-wide traversal with per-lane refill (trace_core.h). The closest-hit queue and the any-hit
+// queue form one index range [0, nc + na) drawn by one work counter. Every lane holds its own ray
+// and advances it by one step per loop iteration; a finished lane idles until `refill` or more
+// lanes of its wave are idle (or the whole wave is), when the wave hands new rays to the idle
+// lanes in lane order. Lanes of one wave may hold closest and any-hit rays of different scenes at
+// once. kQ: every scene of the launch has GpuNodeQ nodes (else every one has GpuNode4 nodes).
+// kOne: every job traces one scene (R.nodes1), whose arrays stay in scalar registers and are
+// addressed with 32-bit offsets.
 template <bool kCount, bool kQ, bool kOne>
 __global__ __launch_bounds__(kBlock, kTraceResidentBlocks) void k_trace_refill(RenderDev R, int L, int buf, int refill,
                                                                                uint32_t claim_rays)
 {
-    __shared__ uint32_t stk[kTraceLds * kBlock];
+    __shared__ __align__(16) uint32_t stk[kTraceLds * kBlock];
     const int lane = threadIdx.x & 63;
-    lu32* my = (lu32*)(stk + threadIdx.x);
-    const int ostride = gridDim.x * kBlock;
-    gu32* ovf = (gu32*)(R.stk_ovf + blockIdx.x * kBlock + threadIdx.x);
+    const QueueOvf ovf{(gu32*)(R.stk_ovf + blockIdx.x * kBlock + threadIdx.x), (int)gridDim.x * kBlock};
     const uint32_t nc = R.counters[4 * L + 0];
     const uint32_t total = nc + R.counters[4 * L + 1];
     uint32_t* work = &R.counters[4 * L + 2];
-    const float kInf = __builtin_inff();
     uint32_t vis_nodes = 0, vis_tris = 0, vis_nodes_any = 0, vis_tris_any = 0;
     bool active = false, any = false, exhausted = false;
     // the wave's reserve: queue entries [rb, re) it has claimed and not yet handed to a lane
-    uint32_t rb = 0, re = 0;
-    f3 o = mk(0.f, 0.f, 0.f), d = mk(0.f, 0.f, 0.f);
-    float ix = 0.f, iy = 0.f, iz = 0.f, ox = 0.f, oy = 0.f, oz = 0.f, tmin = 0.f, tcur = 0.f, hb1 = 0.f, hb2 = 0.f;
-    int prim = -1, sp = 0;
-    uint32_t node = 0, own = 0, top = 0;
-    // the last visit's hit leaf children still to test (bit c: child c, tested in child order,
-    // triangle loff of the lowest one next) with that node's refs and counts, and its internal
-    // children (key = entry distance, kInf if missed), not yet culled and pushed while !sorted
-    uint32_t lmask = 0u;
-    int loff = 0, lr0 = 0, lr1 = 0, lr2 = 0, lr3 = 0, lc0 = 0, lc1 = 0, lc2 = 0, lc3 = 0;
-    float key[4] = {0.f, 0.f, 0.f, 0.f};
-    uint32_t id[4] = {0u, 0u, 0u, 0u};
-    bool sorted = true;
+    uint32_t rb = 0, re = 0, own = 0;
+    LaneRay r{};
     const float4* nodes = kOne ? R.nodes1 : nullptr;
     const float4* tris = kOne ? R.tris1 : nullptr;
     for (;;)
@@ -559,25 +524,7 @@ __global__ __launch_bounds__(kBlock, kTraceResidentBlocks) void k_trace_refill(R
                         nodes = R.jobs[job].s.nodes;
                         tris = R.jobs[job].s.tris;
                     }
-                    o = mk(a.x, a.y, a.z);
-                    d = mk(b.x, b.y, b.z);
-                    const float dx = fabsf(d.x) < 1e-20f ? copysignf(1e-20f, d.x) : d.x;
-                    const float dy = fabsf(d.y) < 1e-20f ? copysignf(1e-20f, d.y) : d.y;
-                    const float dz = fabsf(d.z) < 1e-20f ? copysignf(1e-20f, d.z) : d.z;
-                    ix = 1.f / dx;
-                    iy = 1.f / dy;
-                    iz = 1.f / dz;
-                    ox = o.x * ix;
-                    oy = o.y * iy;
-                    oz = o.z * iz;
-                    tmin = a.w;
-                    tcur = b.w;
-                    prim = -1;
-                    hb1 = hb2 = 0.f;
-                    node = 0;
-                    sp = 0;
-                    lmask = 0u;
-                    sorted = true;
+                    start_ray<kBlock>(r, stk, a, b);
                     active = true;
                 }
             }
@@ -593,105 +540,20 @@ __global__ __launch_bounds__(kBlock, kTraceResidentBlocks) void k_trace_refill(R
         }
         if (__ballot(active) == 0ull) break;
         if (!active) continue;
-        // ---- one step: a triangle of the pending leaves, then, once a lane's leaves are
-        // done, its node's internal children and the next node's visit ----
-        // A visit's leaf triangles are tested one per iteration, before its internal children
-        // are culled against the updated tcur, sorted and pushed (the order traverse4 tests and
-        // culls in); a lane whose last leaf triangle, or whose stack pop, settles its next
-        // node visits that node in the same iteration. A wave so runs a triangle test, a sort
-        // and a visit per iteration over whichever of its lanes need them, instead of looping
-        // over its busiest lane's triangles while the other lanes wait.
-        bool done = false;
-        if (lmask)
+        uint32_t nv = 0, tv = 0;
+        const bool done = step4<kCount, kQ, kOne, kTraceLds, kBlock>(r, any, nodes, tris, stk, ovf, nv, tv);
+        if (kCount)
         {
-            const int c = __builtin_ctz(lmask);
-            const int lref = c == 0 ? lr0 : c == 1 ? lr1 : c == 2 ? lr2 : lr3;
-            const int lcnt = c == 0 ? lc0 : c == 1 ? lc1 : c == 2 ? lc2 : lc3;
-            const int tq = lref + loff;
-            const float4 v0 = gload(tris, 3 * (size_t)tq + 0);
-            const float4 a1 = gload(tris, 3 * (size_t)tq + 1);
-            const float4 a2 = gload(tris, 3 * (size_t)tq + 2);
-            if (kCount) (any ? vis_tris_any : vis_tris)++;
-            float t, u, v;
-            if (intersect_face(ld3(v0), ld3(a1), ld3(a2), o, d, tmin, tcur, t, u, v))
-            {
-                prim = __builtin_bit_cast(int, v0.w);
-                tcur = t;
-                hb1 = u;
-                hb2 = v;
-                if (any) done = true;
-            }
-            if (++loff == lcnt)
-            {
-                lmask &= lmask - 1u;
-                loff = 0;
-            }
-        }
-        if (!done && !sorted && lmask == 0u)
-        {
-            // internal children still in front of the (possibly updated) closest hit, nearest
-            // first: visit it, push the others
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (!(key[c] <= tcur)) key[c] = kInf;
-#define BSH_CSWAP(a, b)                                       \
-    if (key[b] < key[a])                                      \
-    {                                                         \
-        float tk = key[a]; key[a] = key[b]; key[b] = tk;      \
-        uint32_t ti = id[a]; id[a] = id[b]; id[b] = ti;       \
-    }
-            BSH_CSWAP(0, 1)
-            BSH_CSWAP(2, 3)
-            BSH_CSWAP(0, 2)
-            BSH_CSWAP(1, 3)
-            BSH_CSWAP(1, 2)
-#undef BSH_CSWAP
-            const int n = (key[0] < kInf) + (key[1] < kInf) + (key[2] < kInf) + (key[3] < kInf);
-            if (n == 0)
-            {
-                if (sp == 0) done = true;
-                else node = pop_top(my, ovf, ostride, sp, top);
-            }
-            else
-            {
-#pragma unroll
-                for (int k = 3; k >= 1; --k)
-                    if (k < n) push_top(my, ovf, ostride, sp, top, id[k]);
-                node = id[0];
-            }
-            sorted = true;
-        }
-        if (!done && sorted && lmask == 0u)
-        {
-            // visit the next node; its internal children are sorted in the next iteration,
-            // after its leaf triangles
-            if (kCount) (any ? vis_nodes_any : vis_nodes)++;
-            int ref[4], cn[4];
-            float tn[4];
-            bool hitc[4];
-            node4_test<kQ>(nodes, node, ix, iy, iz, ox, oy, oz, tmin, tcur, tn, hitc, ref, cn);
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-            {
-                key[c] = (hitc[c] && cn[c] == 0) ? tn[c] : kInf;
-                id[c] = (uint32_t)ref[c];
-            }
-            // the hit leaf children, tested from the next iteration on
-            lmask = 0u;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) lmask |= (hitc[c] && cn[c] > 0) ? 1u << c : 0u;
-            loff = 0;
-            lr0 = ref[0]; lr1 = ref[1]; lr2 = ref[2]; lr3 = ref[3];
-            lc0 = cn[0]; lc1 = cn[1]; lc2 = cn[2]; lc3 = cn[3];
-            sorted = false;
+            (any ? vis_nodes_any : vis_nodes) += nv;
+            (any ? vis_tris_any : vis_tris) += tv;
         }
         if (done)
         {
             const uint32_t kind = own >> 29, idx = own & ((1u << 29) - 1u);
-            if (any) R.nee_res[idx] = make_int4(prim >= 0 ? 1 : 0, 0, 0, 0);
+            if (any) R.nee_res[idx] = make_int4(r.prim >= 0 ? 1 : 0, 0, 0, 0);
             else
             {
-                const int4 res = make_int4(prim, __float_as_int(tcur), __float_as_int(hb1), __float_as_int(hb2));
+                const int4 res = make_int4(r.prim, __float_as_int(r.tcur), __float_as_int(r.b1), __float_as_int(r.b2));
                 if (kind == Q_EXT) R.hit[idx] = res;
                 else R.nee_res[idx] = res;
             }
@@ -2095,8 +1957,10 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
         R.pdir = probe_dir ? lw.pdir.p : nullptr;
         R.nodes1 = hjobs.empty() ? nullptr : hjobs[0].s.nodes;
         R.tris1 = hjobs.empty() ? nullptr : hjobs[0].s.tris;
+        // (the single-scene trace kernel addresses both arrays with 32-bit byte offsets)
         for (const JobDev& J : hjobs)
-            if (J.s.nodes != R.nodes1 || J.s.tris != R.tris1) R.nodes1 = R.tris1 = nullptr;
+            if (J.s.nodes != R.nodes1 || J.s.tris != R.tris1 || (uint64_t)J.s.ntris * 64 >= (1ull << 32))
+                R.nodes1 = R.tris1 = nullptr;
         R.rec = record ? lw.rec.p : nullptr;
         R.rec_out = record ? gr->records : nullptr;
         R.rec_cap = record ? (uint32_t)std::min<size_t>(gr->cap, 0xffffffffu) : 0u;
