@@ -60,12 +60,17 @@ constexpr int kTraceLds = 16;
 // Training records are kept for the first kRecVerts vertices of a path, 5 float4 each.
 constexpr int kRecVerts = 4, kRecStride = 5 * kRecVerts;
 static_assert(kGuideSeg == kBlock, "guide row segments are the blocks of k_guide_inputs");
-constexpr int kMaxTraceBlocksPerCU = 5;
-constexpr int kTraceBlocksPerLane = 3;   // the default when two lanes run
-// k_trace_refill's launch bound: registers for 6 workgroups per CU (6 waves per SIMD, at most
-// 80 VGPRs), so both lanes' default grids (3 per CU each) are resident at once whatever the
-// node layout (the quantised layout's decode would otherwise take 89).
-constexpr int kTraceResidentBlocks = 2 * kTraceBlocksPerLane;
+// Persistent trace workgroups per CU by default: 8 on one lane (all that fit at 64 VGPRs), 4 per
+// lane on two. Measured with 3 / 4 / 5 / 6 / 8 (ms): 1080p frame on two lanes 229.3 / 227.0 /
+// 229.2 / 230.0 / 228.5; Cornell 256^2 on one lane 1.28 / 1.21 / 1.18 / 1.17 / 1.16; guided 1024^2
+// pass on one lane 8.91 / 8.49 / 8.27 / 8.16 / 8.09.
+constexpr int kTraceBlocksOneLane = 8;
+constexpr int kTraceBlocksPerLane = 4;
+// k_trace_refill's launch bounds. One scene: 64 VGPRs, 8 workgroups per CU, without spills (80
+// VGPRs and 6 workgroups: frame 247 ms against 235, before the work counters were split). Several
+// scenes: 72 VGPRs, since at 64 the per-lane array pointers spill (batch of 16 scenes 13.0 ms
+// against 10.85; 80 VGPRs 10.87).
+constexpr int kTraceResidentBlocks = 8, kTraceResidentMulti = 7;
 // The shade kernel is held to 128 VGPRs: 4 waves per SIMD (at 129 it would run 3). Holding the
 // plain variant to 5 or 6 waves (96 or 80 VGPRs, 24 or 50 of them spilled) made the 1080p
 // terrain frame 1.1 and 1.5 % slower.
@@ -80,11 +85,15 @@ static_assert(kMaxLaunches > 250, "a job's depth is at most 250, so a chunk has 
 // Measured on the 3M-triangle terrain at 1080p: 8 lanes 733 Mrays/s, 16 1058, 32 1314,
 // 48 1381, 56 1393, 64 1353; whole 64-ray batches per wave (k_trace_queue) 1065.
 constexpr int kDefaultRefill = 56;
-// Queue entries a trace wave claims per atomic on the work counter when the run spans several
-// scenes and the tuning leaves claim_rays 0 (a single scene claims exactly the idle lanes).
-// Measured: 64 seeded scenes (1k-2M triangles) 2875 -> 3193 Mrays/s; on one 3M-triangle
-// scene 128 cost 3 % (the small late-bounce launches lose balance).
-constexpr uint32_t kClaimRays = 128;
+// Work counters of a k_trace_refill launch, each on a cache line of its own; the queue is dealt to
+// them in runs of kWorkRun entries. Returning atomics on one line are served about 6 ns apart, so
+// with one counter a launch of 3M short rays took at least 0.3 ms for its 54,000 claims, whatever
+// the rays cost. Interleaved runs keep all waves in one window of the queue (neighbouring entries
+// share cache lines), and as workgroups are dealt to the 8 XCDs in turn, a part's runs go through
+// one XCD's L2. Measured (ms; Cornell frame / 4096-probe bake / 1080p frame): one counter 2.56 /
+// 7.95 / 235.5; 16 parts of 256 entries 1.17 / 7.39 / 227.9, 1024 1.17 / 7.12 / 228.1, 2048 1.16 /
+// 7.09 / 226.0, 16384 1.18 / 7.38 / 227.0; 8 parts 1.23 / 7.11 / 225.9; 32 parts 1.17 / 7.13 / 227.3.
+constexpr uint32_t kWorkParts = 16, kWorkRun = 2048, kWorkStride = 32;
 // A single-chunk run at least this large is split in two for the two wavefront lanes.
 constexpr size_t kSplitPaths = (size_t)1 << 22;
 
@@ -114,8 +123,9 @@ struct RenderDev
     float4 *qc_o[2], *qc_d[2], *qa_o[2], *qa_d[2];
     int *qc_own[2], *qa_own[2];
     uint32_t* counters;            // per launch L: closest count, any count (one 64-bit word, so a
-                                   // shade wave claims both with one atomic), closest or joint work,
-                                   // any work
+                                   // shade wave claims both with one atomic), closest work, any work
+                                   // (k_trace_queue)
+    uint32_t* work;                // per launch L: kWorkParts work counters, kWorkStride apart (k_trace_refill)
     uint32_t* alive[2];            // live paths: shade b reads list b & 1, writes list (b + 1) & 1
     uint32_t* alive_n;             // per bounce: length of its live-path list (b >= 1)
     unsigned long long* stats;     // closest, any, node visits, triangle tests, then kRowParts guided-row partials
@@ -455,13 +465,18 @@ __global__ __launch_bounds__(kBlock) void k_trace_queue(RenderDev R, int L, int 
 // The overflow slots of a trace thread's stack: entries past kTraceLds, [entry][trace thread].
 struct QueueOvf
 {
-    gu32* p;
-    int stride;
-    __device__ __forceinline__ gu32& at(int i) const { return p[(size_t)i * stride]; }
+    uint32_t* p;
+    __device__ __forceinline__ gu32& at(int i) const
+    {
+        // opaque, so that the slot's address is formed where it is used, not kept in registers
+        uint32_t t = threadIdx.x;
+        asm volatile("" : "+v"(t));
+        return ((gu32*)p)[((size_t)i * gridDim.x + blockIdx.x) * kBlock + t];
+    }
 };
 
 // 4-wide traversal with per-lane refill (trace_core.h). The closest-hit queue and the any-hit
-// queue form one index range [0, nc + na) drawn by one work counter. Every lane holds its own ray
+// queue form one index range [0, nc + na), dealt in runs to kWorkParts work counters. Every lane holds its own ray
 // and advances it by one step per loop iteration; a finished lane idles until `refill` or more
 // lanes of its wave are idle (or the whole wave is), when the wave hands new rays to the idle
 // lanes in lane order. Lanes of one wave may hold closest and any-hit rays of different scenes at
@@ -469,15 +484,20 @@ struct QueueOvf
 // kOne: every job traces one scene (R.nodes1), whose arrays stay in scalar registers and are
 // addressed with 32-bit offsets.
 template <bool kCount, bool kQ, bool kOne>
-__global__ __launch_bounds__(kBlock, kTraceResidentBlocks) void k_trace_refill(RenderDev R, int L, int buf, int refill,
-                                                                               uint32_t claim_rays)
+__global__ __launch_bounds__(kBlock, kOne && !kCount ? kTraceResidentBlocks : kTraceResidentMulti) void
+k_trace_refill(RenderDev R, int L, int buf, int refill, uint32_t claim_rays)
 {
     __shared__ __align__(16) uint32_t stk[kTraceLds * kBlock];
     const int lane = threadIdx.x & 63;
-    const QueueOvf ovf{(gu32*)(R.stk_ovf + blockIdx.x * kBlock + threadIdx.x), (int)gridDim.x * kBlock};
+    const QueueOvf ovf{R.stk_ovf};
     const uint32_t nc = R.counters[4 * L + 0];
-    const uint32_t total = nc + R.counters[4 * L + 1];
-    uint32_t* work = &R.counters[4 * L + 2];
+    const uint32_t part = blockIdx.x % kWorkParts;
+    uint32_t* work = &R.work[((uint32_t)L * kWorkParts + part) * kWorkStride];
+    // entries of this part: position p is queue entry (p / kWorkRun * kWorkParts + part) * kWorkRun +
+    // p % kWorkRun
+    const uint32_t all = nc + R.counters[4 * L + 1], last = all % (kWorkRun * kWorkParts);
+    const uint32_t total = all / (kWorkRun * kWorkParts) * kWorkRun +
+                           min(kWorkRun, last - min(last, part * kWorkRun));
     uint32_t vis_nodes = 0, vis_tris = 0, vis_nodes_any = 0, vis_tris_any = 0;
     bool active = false, any = false, exhausted = false;
     // the wave's reserve: queue entries [rb, re) it has claimed and not yet handed to a lane
@@ -489,9 +509,7 @@ __global__ __launch_bounds__(kBlock, kTraceResidentBlocks) void k_trace_refill(R
     {
         // ---- refill the idle lanes (wave-uniform decision) ----
         // Idle lanes take entries from the reserve first. A wave whose reserve is short claims
-        // claim_rays more with one atomic (0: exactly its idle lanes, so no reserve is kept):
-        // with many small scenes, whose rays finish fast, the counter then sees a fraction of
-        // the refills, and a wave still takes its rays in queue order.
+        // claim_rays more with one atomic (0: exactly its idle lanes, so no reserve is kept).
         const unsigned long long idle = __ballot(!active);
         const uint32_t nidle = (uint32_t)__popcll(idle);
         if ((!exhausted || rb < re) && (nidle >= (uint32_t)refill || nidle == 64u))
@@ -510,9 +528,10 @@ __global__ __launch_bounds__(kBlock, kTraceResidentBlocks) void k_trace_refill(R
             if (!active)
             {
                 const uint32_t rank = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                const uint32_t q = rank < from_res ? rb + rank : claim ? nb + (rank - from_res) : total;
-                if (q < total)
+                const uint32_t p = rank < from_res ? rb + rank : claim ? nb + (rank - from_res) : total;
+                if (p < total)
                 {
+                    const uint32_t q = (p / kWorkRun * kWorkParts + part) * kWorkRun + p % kWorkRun;
                     any = q >= nc;
                     const uint32_t k = any ? q - nc : q;
                     const float4 a = gload(any ? R.qa_o[buf] : R.qc_o[buf], k);
@@ -1562,12 +1581,13 @@ static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, c
                                 const std::vector<JobDev>& hjobs, bool count, const bsh_tuning& tune, LaunchTimer* T,
                                 GuideRun* gr)
 {
-    const int trace_blocks = c->num_cus * std::max(1, tune.trace_blocks_per_cu);
+    const int max_blocks = c->num_cus * std::max(1, tune.trace_blocks_per_cu);
     const int refill = tune.refill_lanes == 0 ? kDefaultRefill : tune.refill_lanes;
     const bool one = hjobs.size() == 1;   // every path of the run belongs to job 0
-    // per-atomic trace claims: the tuning's, else exactly the idle lanes on one scene and
-    // kClaimRays when the run's jobs trace several (R.nodes1 is set only for one scene)
-    const uint32_t claim = tune.claim_rays > 0 ? (uint32_t)tune.claim_rays : lanes[0].R.nodes1 ? 0u : kClaimRays;
+    // entries per claim: the tuning's, else exactly the idle lanes (a reserve of 64, 128 or 256
+    // entries per wave: batch of 16 scenes 11.4, 11.6, 11.9 ms against 10.85; 1080p frame 237 ms
+    // with 64 against 228)
+    const uint32_t claim = (uint32_t)tune.claim_rays;
     for (size_t ci = 0; ci < chunks.size(); ++ci)
     {
         const Chunk& ch = chunks[ci];
@@ -1577,6 +1597,10 @@ static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, c
         hipStream_t st = ln.st;
         const int launches = ch.depth + 1;
         R.P = ch.P;
+        // no more trace workgroups than the chunk's rays can use (a bounce has at most one extension
+        // ray and one ray per NEE slot and path), and one for every work counter
+        const size_t most_rays = (size_t)ch.P * (1 + ((size_t)1 << R.Kshift));
+        const int trace_blocks = (int)std::max<size_t>(kWorkParts, std::min<size_t>(max_blocks, (most_rays + kBlock - 1) / kBlock));
         bool full = false, lights = false, wide = refill > 0, qall = true, qany = false;
         for (const Segment& sg : ch.segs)
         {
@@ -1892,12 +1916,9 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     // Two lanes when the run has chunks to alternate and nothing ties the chunks to one order
     // (training records take a running offset).
     const int nlanes = record || tune.lanes == 1 ? 1 : (int)std::min<size_t>(bsh_context::kLanes, chunks.size());
-    // persistent trace workgroups per CU: all of them on one lane; on two lanes each lane's
-    // grid leaves room for the other lane's, which the trace kernel's register bound keeps
-    // resident beside it (1080p frame, 16 chunks: 3 per CU 2515 Mrays/s, 4 2483, 5 2468, 2 2415;
-    // 4096-probe bake, two chunks side by side: 3 per CU 2302-2337, 4 2244-2250, 5 2232, 2
-    // 2084-2091)
-    if (tune.trace_blocks_per_cu <= 0) tune.trace_blocks_per_cu = nlanes > 1 ? kTraceBlocksPerLane : kMaxTraceBlocksPerCU;
+    // persistent trace workgroups per CU: all that fit on one lane; on two lanes each lane's grid
+    // leaves room for the other lane's kernels
+    if (tune.trace_blocks_per_cu <= 0) tune.trace_blocks_per_cu = nlanes > 1 ? kTraceBlocksPerLane : kTraceBlocksOneLane;
     for (int k = 0; k + 1 < nlanes; ++k)
         if (!c->lane_stream[k]) BSH_HIP(hipStreamCreateWithFlags(&c->lane_stream[k], hipStreamNonBlocking));
     bool probe_dir = false;
@@ -1905,7 +1926,9 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     // 4 queue counters per launch, then, from the next 256-B boundary (a cache line of their
     // own), the live-path counts of bounces 0 .. maxdepth + 1; every chunk clears the buffer
     const size_t alive_off = ((size_t)4 * (maxdepth + 1) + 63) / 64 * 64;
-    const size_t trace_threads = (size_t)c->num_cus * std::max(1, tune.trace_blocks_per_cu) * kBlock;
+    // (then, from a further 256-B boundary, the trace launches' work counters)
+    const size_t work_off = (alive_off + maxdepth + 2 + 63) / 64 * 64;
+    const size_t trace_threads = std::max<size_t>((size_t)c->num_cus * std::max(1, tune.trace_blocks_per_cu), kWorkParts) * kBlock;
     BSH_HIP(c->jobs.alloc(hjobs.size()));
     BSH_HIP(hipMemcpyAsync(c->jobs.p, hjobs.data(), hjobs.size() * sizeof(JobDev), hipMemcpyHostToDevice, st));
     BSH_TRY(ensure_work(c->work, P, K, nlmax));   // lane 0's buffers also hold the run's statistics
@@ -1914,7 +1937,7 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     // every lane's buffers and device view (the statistics are lane 0's, shared)
     auto setup_lane = [&](RenderWork& lw, RenderDev& R) -> bsh_status {
         BSH_TRY(ensure_work(lw, P, K, nlmax));
-        BSH_HIP(lw.counters.alloc(alive_off + maxdepth + 2));
+        BSH_HIP(lw.counters.alloc(work_off + (size_t)(maxdepth + 1) * kWorkParts * kWorkStride));
         if (guided)
         {
             const size_t Pb = (P + kBlock - 1) / kBlock * kBlock;   // rows live in whole segments
@@ -1945,6 +1968,7 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
         }
         R.counters = lw.counters.p;
         R.alive_n = lw.counters.p + alive_off;
+        R.work = lw.counters.p + work_off;
         R.alive[0] = lw.alive[0].p;
         R.alive[1] = lw.alive[1].p;
         R.stats = w.stats.p;

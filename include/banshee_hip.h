@@ -394,10 +394,8 @@ bsh_status bsh_sh_irradiance(bsh_context* ctx, int lmax, const float* coeffs, co
    ray and a wave claims new rays once this many of its 64 lanes are idle (1..64; 0 = the
    default, 56); -1 traces in whole 64-ray batches per wave instead (also the form used when
    a chunk holds a binary BVH). claim_rays: queue entries a trace wave claims per atomic on
-   the launch's work counter, keeping what its idle lanes do not take for its next refills
-   (64..4096; 0 = automatic: exactly the idle lanes when every job of the run shares one
-   scene, 128 when the run spans several, whose small scenes refill often enough for the
-   shared counter to limit). Results do not depend on refill_lanes or claim_rays. */
+   one of the launch's work counters, keeping what its idle lanes do not take for its next
+   refills (64..4096; 0 = exactly the idle lanes). Results do not depend on refill_lanes or claim_rays. */
 typedef struct
 {
     int32_t paths_per_chunk;
