@@ -303,6 +303,25 @@ __device__ __forceinline__ void node4_test(const float4* nodes, uint32_t node, f
     }
 }
 
+// A child's entry distance and node index as the high and low word of a double.
+__device__ __forceinline__ double key_pair(float key, uint32_t id) { return __hiloint2double(__float_as_int(key), (int)id); }
+__device__ __forceinline__ float pair_key(double k) { return __int_as_float(__double2hiint(k)); }
+__device__ __forceinline__ uint32_t pair_id(double k) { return (uint32_t)__double2loint(k); }
+
+// Compare-exchange of (key, id) pairs as doubles, by key, then by id: the order in which every
+// 4-wide traversal visits a node's children, so a tie between triangles at the same distance is
+// resolved alike by all of them. Keys are finite floats or
+// +inf, whose patterns are finite as the high word of a double, so the order is the keys'.
+// (Instructions written out: fmin / fmax would first canonicalise both operands.)
+__device__ __forceinline__ void pair_sort2(double& a, double& b)
+{
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
+}
+
 // 4-wide traversal over GpuNode4 or GpuNodeQ: one visit loads the node (128 or 64 B), tests four boxes,
 // intersects leaf children at once, then visits the hit internal children nearest first
 // (a 5-comparator sorting network on their entry distances; the far ones are pushed,
@@ -363,27 +382,16 @@ __device__ __forceinline__ bool traverse4(const SceneDev& s, f3 o, f3 d, float t
                 hit[c] = false;
             }
         }
-        float key[4];
-        uint32_t id[4];
+        double k[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-        {
-            key[c] = (hit[c] && tn[c] <= tcur) ? tn[c] : kInf;
-            id[c] = (uint32_t)ref[c];
-        }
-#define BSH_CSWAP(a, b)                                       \
-    if (key[b] < key[a])                                      \
-    {                                                         \
-        float tk = key[a]; key[a] = key[b]; key[b] = tk;      \
-        uint32_t ti = id[a]; id[a] = id[b]; id[b] = ti;       \
-    }
-        BSH_CSWAP(0, 1)
-        BSH_CSWAP(2, 3)
-        BSH_CSWAP(0, 2)
-        BSH_CSWAP(1, 3)
-        BSH_CSWAP(1, 2)
-#undef BSH_CSWAP
-        const int n = (key[0] < kInf) + (key[1] < kInf) + (key[2] < kInf) + (key[3] < kInf);
+        for (int c = 0; c < 4; ++c) k[c] = key_pair((hit[c] && tn[c] <= tcur) ? tn[c] : kInf, (uint32_t)ref[c]);
+        pair_sort2(k[0], k[1]);
+        pair_sort2(k[2], k[3]);
+        pair_sort2(k[0], k[2]);
+        pair_sort2(k[1], k[3]);
+        pair_sort2(k[1], k[2]);
+        const int n = (pair_key(k[0]) < kInf) + (pair_key(k[1]) < kInf) + (pair_key(k[2]) < kInf) +
+                      (pair_key(k[3]) < kInf);
         if (n == 0)
         {
             if (sp == 0) break;
@@ -391,9 +399,9 @@ __device__ __forceinline__ bool traverse4(const SceneDev& s, f3 o, f3 d, float t
             continue;
         }
 #pragma unroll
-        for (int k = 3; k >= 1; --k)
-            if (k < n) stack_push<kLds, kMaxStack4>((lu32*)stk, stride, (gu32*)ovf, ostride, sp, id[k]);
-        node = id[0];
+        for (int j = 3; j >= 1; --j)
+            if (j < n) stack_push<kLds, kMaxStack4>((lu32*)stk, stride, (gu32*)ovf, ostride, sp, pair_id(k[j]));
+        node = pair_id(k[0]);
     }
     res.prim = prim;
     res.t = tcur;

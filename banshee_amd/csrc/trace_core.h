@@ -70,22 +70,6 @@ __device__ __forceinline__ bool intersect_face_dev(f3 p1, f3 e1, f3 e2, f3 o, f3
     return false;
 }
 
-__device__ __forceinline__ double key_pair(float key, uint32_t id) { return __hiloint2double(__float_as_int(key), (int)id); }
-__device__ __forceinline__ float pair_key(double k) { return __int_as_float(__double2hiint(k)); }
-__device__ __forceinline__ uint32_t pair_id(double k) { return (uint32_t)__double2loint(k); }
-
-// Compare-exchange of (key, id) pairs as doubles, by key, then by id. Keys are finite floats or
-// +inf, whose patterns are finite as the high word of a double, so the order is the keys'.
-// (Instructions written out: fmin / fmax would first canonicalise both operands.)
-__device__ __forceinline__ void pair_sort2(double& a, double& b)
-{
-    double lo, hi;
-    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
-    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
-    a = lo;
-    b = hi;
-}
-
 // A lane's ray and traversal state.
 struct LaneRay
 {
