@@ -186,6 +186,8 @@ struct bsh_context
             if (s) (void)hipStreamDestroy(s);
     }
     bsh::DevBuf<bsh::JobDev> jobs;
+    std::mutex env_mu;             // guards env_part, the partial sums of an environment projection
+    bsh::DevBuf<float> env_part;
     bsh_tuning tuning{1 << 23, 0, 0, 0, 0, 0};
     bsh_render_stats stats{};
     std::vector<bsh_launch_stats> launch_stats;   // per bounce launch, of the last run

@@ -15,73 +15,122 @@
 namespace bsh {
 
 constexpr int kShBlock = 256;
+// Blocks of the environment projection: two per CU.
+constexpr int kEnvMaxBlocks = 512;
+// The context's scratch for it (128 KB at lmax 4 and a map up to kEnvMaxBlocks x 256 columns wide,
+// and some more for maps whose rows need more blocks).
+constexpr size_t kEnvCtxFloats = (size_t)2 * kEnvMaxBlocks * 3 * kShMaxTerms;
 
-// Pass 1: each block sums the contributions of kShBlock consecutive texels, in the
-// reference's loop order (phi outer, theta inner), with a fixed LDS tree.
+// Environment projection: c_i = sum over the map's cells of e Y_i(w) sin(theta) (pi / H) (2 pi / W).
+// Pass 1: a block takes a tile of kShTile columns (phi; the columns of a narrower map in several
+// rows at a time) and `rows` rows (theta); each thread keeps its column and sums its rows' terms in
+// registers, then the block adds its threads' sums in LDS, one channel at a time, in a fixed order.
+// Bound by the map's 12 B per cell, then by the basis (about 60 instructions per cell at lmax 2).
+// Lanes read consecutive texels (the loop order of the reference, theta inner, put them a map row
+// apart), and the block reduces once per coefficient and 256 threads, not with eight barriers per
+// coefficient and 256 cells: 2048 x 1024, lmax 2: 88 -> 13 us, and pass 2, whose one block walked
+// 8192 partial sums per coefficient, 1634 -> 4 us; the call, which also filled its angle tables on
+// the host and allocated, with 262,144 irradiances 1773 -> 33 us.
+constexpr int kShTile = 256;
 template <int LMAX>
-__global__ __launch_bounds__(kShBlock) void k_env_partial(const float* env, int W, int H, const float* sinth,
-                                                        const float* costh, const float* sinph, const float* cosph,
-                                                        float* partial)
+__global__ __launch_bounds__(kShBlock) void k_env_partial(const float* __restrict__ env, int W, int H, int cols, int rows,
+                                                        float* __restrict__ partial)
 {
     constexpr int NT = (LMAX + 1) * (LMAX + 1);
-    __shared__ float red[kShBlock];
-    int k = blockIdx.x * kShBlock + threadIdx.x;
+    constexpr int kPitch = kShBlock + 1;
+    __shared__ float red[NT * kPitch];
+    __shared__ float s_sin[kShBlock], s_cos[kShBlock], s_w[kShBlock];
+    const int t = threadIdx.x;
+    // the angles in float as the reference forms them (shproject.cpp:85-104), their sines and
+    // cosines rounded from double
+    const float thetastep = kPi / H, phistep = 2.f * kPi / W;
+    const float theta0 = kPi / H / 2, phi0 = 2.f * kPi / W / 2;
+    const int nx = (W + cols - 1) / cols, bx = blockIdx.x % nx;
+    const int row0 = blockIdx.x / nx * rows, row1 = min(row0 + rows, H);
+    if (row0 + t < row1)
+    {
+        const double a = (double)(theta0 + (float)(row0 + t) * thetastep);
+        s_sin[t] = (float)sin(a);
+        s_cos[t] = (float)cos(a);
+        s_w[t] = s_sin[t] * thetastep * phistep;
+    }
+    __syncthreads();
+    const int phi = bx * cols + t % cols, sub = t / cols, nsub = kShBlock / cols;
     float c[3 * NT];
 #pragma unroll
     for (int i = 0; i < 3 * NT; ++i) c[i] = 0.f;
-    if (k < W * H)
+    if (phi < W && sub < nsub)
     {
-        int phi = k / H, theta = k % H;
-        f3 w = normalize(mk(sinth[theta] * cosph[phi], costh[theta], sinth[theta] * sinph[phi]));
-        float ux = (float)phi / W, uy = (float)theta / H;
-        int iu = (int)floorf(ux * W), iv = (int)floorf(uy * H);
-        const float* e = env + 3 * ((size_t)W * iv + iu);
-        float y[kShMaxTerms];
-        sh_evaluate(w, LMAX, y);
-        float a = kPi / H, b = 2.f * kPi / W;
+        const double a = (double)(phi0 + (float)phi * phistep);
+        const float sp = (float)sin(a), cp = (float)cos(a);
+        const int iu = (int)floorf((float)phi / W * W);
+#pragma unroll 4
+        for (int r = row0 + sub; r < row1; r += nsub)
+        {
+            const int iv = (int)floorf((float)r / H * H);
+            const float* e = env + 3 * ((size_t)W * iv + iu);
+            const float st = s_sin[r - row0], ct = s_cos[r - row0], w = s_w[r - row0];
+            const float ex = e[0] * w, ey = e[1] * w, ez = e[2] * w;
+            float y[NT];
+            sh_poly<LMAX>(st * cp, ct, st * sp, y);
 #pragma unroll
-        for (int i = 0; i < NT; ++i)
-        {
-            c[3 * i + 0] = e[0] * y[i] * sinth[theta] * a * b;
-            c[3 * i + 1] = e[1] * y[i] * sinth[theta] * a * b;
-            c[3 * i + 2] = e[2] * y[i] * sinth[theta] * a * b;
+            for (int i = 0; i < NT; ++i)
+            {
+                c[3 * i + 0] = __builtin_fmaf(ex, y[i], c[3 * i + 0]);
+                c[3 * i + 1] = __builtin_fmaf(ey, y[i], c[3 * i + 1]);
+                c[3 * i + 2] = __builtin_fmaf(ez, y[i], c[3 * i + 2]);
+            }
         }
     }
-    for (int i = 0; i < 3 * NT; ++i)
+    const int nblocks = gridDim.x, block = blockIdx.x;
+#pragma unroll
+    for (int ch = 0; ch < 3; ++ch)
     {
-        red[threadIdx.x] = c[i];
+#pragma unroll
+        for (int i = 0; i < NT; ++i) red[i * kPitch + t] = c[3 * i + ch];
         __syncthreads();
-        for (int st = kShBlock / 2; st > 0; st >>= 1)
+        // 8 threads per coefficient add 32 sums each, then one another's
+        for (int i = t >> 3; i < NT; i += kShBlock / 8)
         {
-            if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-            __syncthreads();
+            float s = 0.f;
+#pragma unroll 8
+            for (int k = 0; k < kShBlock / 8; ++k) s += red[i * kPitch + 8 * k + (t & 7)];
+            s += __shfl_xor(s, 1);
+            s += __shfl_xor(s, 2);
+            s += __shfl_xor(s, 4);
+            if ((t & 7) == 0) partial[(size_t)(3 * i + ch) * nblocks + block] = s;
         }
-        if (threadIdx.x == 0) partial[(size_t)blockIdx.x * 3 * NT + i] = red[0];
         __syncthreads();
     }
 }
 
-// Pass 2: one thread per coefficient sums the block partials in block order.
-__global__ void k_env_final(const float* partial, int nblocks, int n, float* coeffs)
+// Pass 2: one wave per coefficient and channel adds the blocks' sums in a fixed order.
+__global__ __launch_bounds__(64) void k_env_final(const float* __restrict__ partial, int nblocks, float* coeffs)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    const float* p = partial + (size_t)blockIdx.x * nblocks;
     float s = 0.f;
-    for (int b = 0; b < nblocks; ++b) s += partial[(size_t)b * n + i];
-    coeffs[i] = s;
+    for (int b = threadIdx.x; b < nblocks; b += 64) s += p[b];
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off);
+    if (threadIdx.x == 0) coeffs[blockIdx.x] = s;
 }
 
-__global__ void k_irradiance(int lmax, const float* coeffs, const float* normals, uint32_t n, float* out)
+// lmax as a template argument: the basis stays in registers and its constants are folded (with lmax
+// at run time 262,144 normals took 9.5 us, now 4.1); the operations and their order are the same.
+template <int LMAX>
+__global__ __launch_bounds__(256) void k_irradiance(const float* __restrict__ coeffs, const float* __restrict__ normals,
+                                                    uint32_t n, float* __restrict__ out)
 {
     uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    int nt = (lmax + 1) * (lmax + 1);
     float y[kShMaxTerms];
-    sh_evaluate(mk(normals[3 * t], normals[3 * t + 1], normals[3 * t + 2]), lmax, y);
+    sh_evaluate(mk(normals[3 * (size_t)t], normals[3 * (size_t)t + 1], normals[3 * (size_t)t + 2]), LMAX, y);
     f3 e = mk(0.f, 0.f, 0.f);
-    for (int l = 0; l <= lmax; ++l)
+#pragma unroll
+    for (int l = 0; l <= LMAX; ++l)
     {
         float lam = sh_lambda(l);
+#pragma unroll
         for (int m = -l; m <= l; ++m)
         {
             int o = sh_index(l, m);
@@ -90,10 +139,9 @@ __global__ void k_irradiance(int lmax, const float* coeffs, const float* normals
             e = e + y[o] * cc * (0.7f / 3.14159265358979323846f);
         }
     }
-    (void)nt;
-    out[3 * t] = e.x;
-    out[3 * t + 1] = e.y;
-    out[3 * t + 2] = e.z;
+    out[3 * (size_t)t] = e.x;
+    out[3 * (size_t)t + 1] = e.y;
+    out[3 * (size_t)t + 2] = e.z;
 }
 
 __global__ void k_diag_sh(int lmax, uint32_t n, const float* dirs, float* out)
@@ -106,27 +154,29 @@ __global__ void k_diag_sh(int lmax, uint32_t n, const float* dirs, float* out)
     for (int i = 0; i < nt; ++i) out[(size_t)t * nt + i] = y[i];
 }
 
-// The sin/cos tables exactly as the reference computes them on the host
-// (shproject.cpp:85-104), laid out as sin(theta)[H], cos(theta)[H], sin(phi)[W], cos(phi)[W];
-// writes entries [first, first + n) of that concatenation.
-static void env_tables(int W, int H, size_t first, size_t n, float* out)
+// Tiling of a map: `cols` columns and `rows` rows per block, about two blocks per CU where the map
+// is large enough and at most kEnvMaxBlocks.
+struct EnvTiles
 {
-    float thetastep = kPi / H, phistep = 2.f * kPi / W;
-    float theta0 = kPi / H / 2, phi0 = 2.f * kPi / W / 2;
-    for (size_t k = 0; k < n; ++k)
-    {
-        size_t i = first + k;
-        if (i < (size_t)H) out[k] = std::sin(theta0 + (int)i * thetastep);
-        else if (i < 2 * (size_t)H) out[k] = std::cos(theta0 + (int)(i - H) * thetastep);
-        else if (i < 2 * (size_t)H + W) out[k] = std::sin(phi0 + (int)(i - 2 * H) * phistep);
-        else out[k] = std::cos(phi0 + (int)(i - 2 * H - W) * phistep);
-    }
+    int cols, rows, nx, ny;
+};
+static EnvTiles env_tiles(int W, int H)
+{
+    EnvTiles t;
+    t.cols = 1;
+    while (t.cols < W && t.cols < kShTile) t.cols *= 2;
+    t.nx = (int)(((int64_t)W + t.cols - 1) / t.cols);
+    const int sub = kShBlock / t.cols;   // rows a block reads at a time
+    const int want = std::max(1, kEnvMaxBlocks / t.nx);
+    t.rows = std::max(sub, (H + want - 1) / want);
+    t.rows = std::min(t.rows, kShBlock);   // a block's angle table
+    t.ny = (H + t.rows - 1) / t.rows;
+    return t;
 }
-
 static size_t env_partial_floats(int W, int H, int lmax)
 {
-    size_t nb = ((size_t)W * H + kShBlock - 1) / kShBlock;
-    return nb * 3 * (lmax + 1) * (lmax + 1);
+    const EnvTiles t = env_tiles(W, H);
+    return (size_t)t.nx * t.ny * 3 * (lmax + 1) * (lmax + 1);
 }
 
 static bsh_status check_env_args(bsh_context* ctx, const float* env, int width, int height, int lmax,
@@ -140,24 +190,22 @@ static bsh_status check_env_args(bsh_context* ctx, const float* env, int width, 
     return BSH_OK;
 }
 
-// Both passes over `tab` (the four tables, 2(W+H) floats) and `partial` (one block's
-// 3(lmax+1)^2 sums per kShBlock texels, every entry written by pass 1 before pass 2 reads it).
-static hipError_t launch_env_projection(const float* env, int W, int H, int lmax, const float* tab, float* partial,
-                                        float* coeffs, hipStream_t st)
+// Both passes; `partial` holds env_partial_floats(W, H, lmax) floats, every one written by pass 1.
+static hipError_t launch_env_projection(const float* env, int W, int H, int lmax, float* partial, float* coeffs,
+                                        hipStream_t st)
 {
-    const float *sth = tab, *cth = tab + H, *sph = tab + 2 * H, *cph = tab + 2 * H + W;
-    int nt3 = 3 * (lmax + 1) * (lmax + 1);
-    int nb = (int)(((size_t)W * H + kShBlock - 1) / kShBlock);
-    dim3 g(nb), b(kShBlock);
+    const EnvTiles q = env_tiles(W, H);
+    const dim3 g((uint32_t)(q.nx * q.ny)), b(kShBlock);
     switch (lmax)
     {
-    case 0: hipLaunchKernelGGL(k_env_partial<0>, g, b, 0, st, env, W, H, sth, cth, sph, cph, partial); break;
-    case 1: hipLaunchKernelGGL(k_env_partial<1>, g, b, 0, st, env, W, H, sth, cth, sph, cph, partial); break;
-    case 2: hipLaunchKernelGGL(k_env_partial<2>, g, b, 0, st, env, W, H, sth, cth, sph, cph, partial); break;
-    case 3: hipLaunchKernelGGL(k_env_partial<3>, g, b, 0, st, env, W, H, sth, cth, sph, cph, partial); break;
-    default: hipLaunchKernelGGL(k_env_partial<4>, g, b, 0, st, env, W, H, sth, cth, sph, cph, partial); break;
+    case 0: hipLaunchKernelGGL(k_env_partial<0>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
+    case 1: hipLaunchKernelGGL(k_env_partial<1>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
+    case 2: hipLaunchKernelGGL(k_env_partial<2>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
+    case 3: hipLaunchKernelGGL(k_env_partial<3>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
+    default: hipLaunchKernelGGL(k_env_partial<4>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
     }
-    hipLaunchKernelGGL(k_env_final, dim3(1), dim3(128), 0, st, partial, nb, nt3, coeffs);
+    hipLaunchKernelGGL(k_env_final, dim3(3 * (lmax + 1) * (lmax + 1)), dim3(64), 0, st, (const float*)partial,
+                       q.nx * q.ny, coeffs);
     return hipGetLastError();
 }
 
@@ -203,14 +251,24 @@ bsh_status bsh_sh_project_env(bsh_context* ctx, const float* env, int width, int
     if (v != BSH_OK) return v;
     BSH_HIP(hipSetDevice(ctx->device));
     hipStream_t st = (hipStream_t)stream;
-    std::vector<float> tab(2 * ((size_t)width + height));
-    env_tables(width, height, 0, tab.size(), tab.data());
-    DevBuf<float> d_tab, d_part;
-    BSH_HIP(d_tab.alloc(tab.size()));
-    BSH_HIP(hipMemcpyAsync(d_tab.p, tab.data(), tab.size() * 4, hipMemcpyHostToDevice, st));
-    BSH_HIP(d_part.alloc(env_partial_floats(width, height, lmax)));
-    BSH_HIP(launch_env_projection(env, width, height, lmax, d_tab.p, d_part.p, coeffs, st));
-    BSH_HIP(hipStreamSynchronize(st));   // the temporaries are freed on return
+    // the context's scratch while no other call is using it, else (another thread's call is in
+    // flight, or the map has more blocks than the scratch holds) an allocation of this call's own
+    const size_t need = env_partial_floats(width, height, lmax);
+    std::unique_lock<std::mutex> lk(ctx->env_mu, std::try_to_lock);
+    DevBuf<float> own;
+    float* part = nullptr;
+    if (lk.owns_lock() && need <= kEnvCtxFloats)
+    {
+        BSH_HIP(ctx->env_part.alloc(kEnvCtxFloats));
+        part = ctx->env_part.p;
+    }
+    else
+    {
+        BSH_HIP(own.alloc(need));
+        part = own.p;
+    }
+    BSH_HIP(launch_env_projection(env, width, height, lmax, part, coeffs, st));
+    BSH_HIP(hipStreamSynchronize(st));   // the sums are read before the scratch is given back
     return BSH_OK;
 }
 
@@ -219,9 +277,11 @@ bsh_status bsh_sh_project_env_noalloc(bsh_context* ctx, const float* env, int wi
 {
     bsh_status v = check_env_args(ctx, env, width, height, lmax, coeffs, "bsh_sh_project_env_noalloc");
     if (v != BSH_OK) return v;
-    size_t ntab = 2 * ((size_t)width + height), npart = env_partial_floats(width, height, lmax);
-    size_t part_off = (ntab + 63) & ~(size_t)63;   // partials start on a 256-B boundary
-    if (part_off + npart > kEnvScratchFloats)
+    // the documented limit: two tables of a map's angles and 3 (lmax + 1)^2 sums per 256 cells
+    const size_t ntab = 2 * ((size_t)width + height);
+    const size_t npart = ((size_t)width * height + 255) / 256 * 3 * (lmax + 1) * (lmax + 1);
+    const size_t part_off = (ntab + 63) & ~(size_t)63;
+    if (part_off + npart > kEnvScratchFloats || env_partial_floats(width, height, lmax) > kEnvScratchFloats)
         return fail(BSH_ERR_INVALID, "bsh_sh_project_env_noalloc: a " + std::to_string(width) + "x" +
                                          std::to_string(height) + " map at lmax " + std::to_string(lmax) + " needs " +
                                          std::to_string((part_off + npart) * 4) + " B of scratch, more than its " +
@@ -231,17 +291,7 @@ bsh_status bsh_sh_project_env_noalloc(bsh_context* ctx, const float* env, int wi
     if (!base) return fail(BSH_ERR_STATE, "bsh_sh_project_env_noalloc: scratch of device " +
                                               std::to_string(ctx->device) + " was not set up by bsh_context_create");
     hipStream_t st = (hipStream_t)stream;
-    // the host tables go up through a fixed stack buffer, one piece at a time; each piece is
-    // waited for before the buffer is refilled
-    float piece[2048];
-    for (size_t o = 0; o < ntab; o += 2048)
-    {
-        size_t n = std::min<size_t>(2048, ntab - o);
-        env_tables(width, height, o, n, piece);
-        BSH_HIP(hipMemcpyAsync(base + o, piece, n * 4, hipMemcpyHostToDevice, st));
-        BSH_HIP(hipStreamSynchronize(st));
-    }
-    BSH_HIP(launch_env_projection(env, width, height, lmax, base, base + part_off, coeffs, st));
+    BSH_HIP(launch_env_projection(env, width, height, lmax, base, coeffs, st));
     return BSH_OK;
 }
 
@@ -252,8 +302,15 @@ bsh_status bsh_sh_irradiance(bsh_context* ctx, int lmax, const float* coeffs, co
     if (lmax < 0 || lmax > kShMaxL) return fail(BSH_ERR_UNSUPPORTED, "bsh_sh_irradiance: lmax must be 0..4");
     if (n == 0) return BSH_OK;
     BSH_HIP(hipSetDevice(ctx->device));
-    hipLaunchKernelGGL(k_irradiance, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, lmax, coeffs,
-                       normals, (uint32_t)n, out);
+    const dim3 g((uint32_t)((n + 255) / 256)), b(256);
+    switch (lmax)
+    {
+    case 0: hipLaunchKernelGGL(k_irradiance<0>, g, b, 0, (hipStream_t)stream, coeffs, normals, (uint32_t)n, out); break;
+    case 1: hipLaunchKernelGGL(k_irradiance<1>, g, b, 0, (hipStream_t)stream, coeffs, normals, (uint32_t)n, out); break;
+    case 2: hipLaunchKernelGGL(k_irradiance<2>, g, b, 0, (hipStream_t)stream, coeffs, normals, (uint32_t)n, out); break;
+    case 3: hipLaunchKernelGGL(k_irradiance<3>, g, b, 0, (hipStream_t)stream, coeffs, normals, (uint32_t)n, out); break;
+    default: hipLaunchKernelGGL(k_irradiance<4>, g, b, 0, (hipStream_t)stream, coeffs, normals, (uint32_t)n, out); break;
+    }
     BSH_HIP(hipGetLastError());
     return BSH_OK;
 }

@@ -84,6 +84,68 @@ BSH_HD void sh_evaluate(f3 p, int lmax, float* coefs)
     }
 }
 
+// ---- the same basis as polynomials ----
+// y_lm = K(l, |m|) Q_lm(z) {Re, Im}(x + i y)^|m|, Q_lm = P_l^m(z) / (1 - z^2)^(m/2): the terms of
+// sh_evaluate without its square roots and divisions, for unit directions and sums that need not
+// round as the reference's do (near the poles, where sh_evaluate loses 1 - z^2 to rounding, the
+// products keep their relative accuracy).
+constexpr double sh_csqrt(double v)
+{
+    double x = v > 1.0 ? v : 1.0;
+    for (int i = 0; i < 60; ++i) x = 0.5 * (x + v / x);
+    return x;
+}
+// K(l, m) (times sqrt 2 where m > 0) and the recurrence's coefficients, formed at compile time.
+struct ShPolyTable
+{
+    float k[kShMaxL + 1][kShMaxL + 1] = {}, a[kShMaxL + 1][kShMaxL + 1] = {}, b[kShMaxL + 1][kShMaxL + 1] = {};
+    constexpr ShPolyTable()
+    {
+        for (int l = 0; l <= kShMaxL; ++l)
+            for (int m = 0; m <= l; ++m)
+            {
+                double f = 1.0;   // (l - m)! / (l + m)!
+                for (int j = l - m + 1; j <= l + m; ++j) f /= j;
+                k[l][m] = (float)((m ? 1.4142135623730951 : 1.0) *
+                                  sh_csqrt((2.0 * l + 1.0) / (4.0 * 3.14159265358979323846) * f));
+                if (l > m)
+                {
+                    a[l][m] = (float)((2.0 * l - 1.0) / (l - m));
+                    b[l][m] = (float)((l - 1.0 + m) / (l - m));
+                }
+            }
+    }
+};
+
+template <int LMAX>
+__device__ __forceinline__ void sh_poly(float x, float y, float z, float (&out)[(LMAX + 1) * (LMAX + 1)])
+{
+    constexpr ShPolyTable T{};
+    float cm = 1.f, sm = 0.f, dfact = 1.f;
+#pragma unroll
+    for (int m = 0; m <= LMAX; ++m)
+    {
+        float q0 = 0.f, q1 = dfact;   // Q_(l-1)m, Q_lm from l = m on
+#pragma unroll
+        for (int l = m; l <= LMAX; ++l)
+        {
+            if (l > m)
+            {
+                const float q = T.a[l][m] * z * q1 - T.b[l][m] * q0;
+                q0 = q1;
+                q1 = q;
+            }
+            const float kq = T.k[l][m] * q1;
+            out[l * l + l + m] = kq * cm;
+            if (m) out[l * l + l - m] = kq * sm;
+        }
+        const float c = cm * x - sm * y;
+        sm = cm * y + sm * x;
+        cm = c;
+        dfact *= -(float)(2 * m + 1);
+    }
+}
+
 // ShConvolveCosTheta table and lambda, sh.cpp:155-180 (lmax <= 4 entries)
 BSH_HD float sh_costheta(int l)
 {
