@@ -79,9 +79,10 @@ struct RenderWork
     DevBuf<float4> ray_o, ray_d, thr, thr_nee, rad, out;
     DevBuf<int4> hit;
     DevBuf<uint4> meta;
-    DevBuf<unsigned long long> nee_mask;   // per path: NEE slots with a ray in flight (bit 2j shadow, 2j+1 MIS)
-    DevBuf<float4> nee_a, nee_b, nee_wi;
-    DevBuf<int4> nee_res;
+    DevBuf<float4> nee_a, nee_wi;      // NEE slots, slot-major
+    DevBuf<float2> nee_b;              // MIS slots
+    DevBuf<int4> nee_res;              // MIS slots
+    DevBuf<uint8_t> nee_occ;           // shadow slots
     DevBuf<float4> qc_o[2], qc_d[2], qa_o[2], qa_d[2];   // closest / any-hit queues
     DevBuf<int> qc_own[2], qa_own[2];
     DevBuf<float4> gin, rec;          // guide network inputs (2 per row), training records (per path)

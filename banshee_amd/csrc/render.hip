@@ -116,10 +116,17 @@ struct RenderDev
     int Kshift;        // NEE slots per path = 1 << Kshift
     float4 *ray_o, *ray_d, *thr, *thr_nee, *rad, *out;
     int4* hit;
-    uint4* meta;       // x: key base, y: flags | bounce << 8 | nee lights << 16 | job << 24, z/w: BSDF sample
-    unsigned long long* nee_mask;   // bit 2j: shadow ray of NEE slot j in flight, 2j + 1: its MIS ray
-    float4 *nee_a, *nee_b, *nee_wi;
-    int4* nee_res;
+    // x: key base, y: flags | bounce << 8 | nee lights << 16 | job << 24, z/w: NEE slots with a ray in
+    // flight (bit 2j: light j's shadow ray, 2j + 1: its MIS ray)
+    uint4* meta;
+    // NEE slot arrays, slot by slot (slot k of path i at k nee_stride + i), so that a bounce touches
+    // dense lines of the slots it uses; those of MIS rays and of shadow rays alone hold half the slots
+    uint32_t nee_stride;
+    float4 *nee_a, *nee_wi;   // per slot: shadow: contribution, direction and distance; MIS: BSDF value
+                              // and cosine, direction and MIS weight
+    float2* nee_b;            // per MIS slot: 1 / pdf, light
+    int4* nee_res;            // per MIS slot: its ray's hit
+    uint8_t* nee_occ;         // per shadow slot: 1 where the ray was blocked
     float4 *qc_o[2], *qc_d[2], *qa_o[2], *qa_d[2];
     int *qc_own[2], *qa_own[2];
     uint32_t* counters;            // per launch L: closest count, any count (one 64-bit word, so a
@@ -313,6 +320,18 @@ __global__ __launch_bounds__(kBlock) void k_raygen_probe(RenderDev R, uint32_t j
     }
 }
 
+__device__ __forceinline__ size_t nee_at(const RenderDev& R, uint32_t slot, uint32_t i)
+{
+    return (size_t)slot * R.nee_stride + i;
+}
+
+// The slot arrays' index of an NEE ray's owner (path << Kshift | slot); half: of the arrays that
+// hold MIS or shadow slots alone.
+__device__ __forceinline__ size_t nee_half(const RenderDev& R, uint32_t idx)
+{
+    return nee_at(R, (idx & ((1u << R.Kshift) - 1u)) >> 1, idx >> R.Kshift);
+}
+
 __device__ __forceinline__ uint32_t path_of(const RenderDev& R, uint32_t kind, uint32_t idx)
 {
     return kind == Q_EXT ? idx : (idx >> R.Kshift);
@@ -437,7 +456,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_queue(RenderDev R, int L, int 
                     int4 o = make_int4(h ? res.prim : -1, __float_as_int(res.t), __float_as_int(res.b1),
                                        __float_as_int(res.b2));
                     if (kind == Q_EXT) R.hit[idx] = o;
-                    else R.nee_res[idx] = o;
+                    else R.nee_res[nee_half(R, idx)] = o;
                 }
                 else
                 {
@@ -446,7 +465,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_queue(RenderDev R, int L, int 
                                                                       b.w, my, kBlock, res, cnt, ovf, ostride)
                                  : traverse<true, kCount, kTraceLds>(S, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w,
                                                                      b.w, my, kBlock, res, cnt, ovf, ostride);
-                    R.nee_res[idx] = make_int4(h ? 1 : 0, 0, 0, 0);
+                    R.nee_occ[nee_half(R, idx)] = h ? 1 : 0;
                 }
                 vis_nodes += cnt.nodes;
                 vis_tris += cnt.tris;
@@ -569,12 +588,12 @@ k_trace_refill(RenderDev R, int L, int buf, int refill, uint32_t claim_rays)
         if (done)
         {
             const uint32_t kind = own >> 29, idx = own & ((1u << 29) - 1u);
-            if (any) R.nee_res[idx] = make_int4(r.prim >= 0 ? 1 : 0, 0, 0, 0);
+            if (any) R.nee_occ[nee_half(R, idx)] = r.prim >= 0 ? 1 : 0;
             else
             {
                 const int4 res = make_int4(r.prim, __float_as_int(r.tcur), __float_as_int(r.b1), __float_as_int(r.b2));
                 if (kind == Q_EXT) R.hit[idx] = res;
-                else R.nee_res[idx] = res;
+                else R.nee_res[nee_half(R, idx)] = res;
             }
             active = false;
         }
@@ -655,32 +674,24 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
             // ---- 1. resolve the NEE rays issued at bounce pb (DiTracer::GetDi tail) ----
             if (fl & F_NEE)
             {
-                const unsigned long long mask = R.nee_mask[i];
+                const unsigned long long mask = (unsigned long long)meta.w << 32 | meta.z;
                 f3 T = ld3(R.thr_nee[i]);
-                f3 ps = ld3(R.ray_o[i]);
                 for (int j = 0; j < ncnt; ++j)
                 {
                     f3 local = mk(0.f, 0.f, 0.f);
-                    size_t ks = (size_t)i * K + 2 * j;
-                    if (mask & (1ull << (2 * j)))
-                    {
-                        if (R.nee_res[ks].x == 0) local = local + ld3(R.nee_a[ks]);
-                    }
+                    const bool shadowed = (mask & (1ull << (2 * j))) && R.nee_occ[nee_at(R, j, i)] != 0;
+                    if ((mask & (1ull << (2 * j))) && !shadowed) local = local + ld3(R.nee_a[nee_at(R, 2 * j, i)]);
                     // a normal-mapped vertex traced two BSDF rays for this light: the one that saw
                     // the normal mapped twice (its light sample was unoccluded, so Evaluate ran
                     // first) in slot 2j + 1, the other in slot 2 ncnt + 2j + 1
                     int bbit = 2 * j + 1;
-                    size_t bks = ks + 1;
-                    if (kLights && (fl & F_NMAP) && (mask & (1ull << (2 * j))) && R.nee_res[ks].x != 0)
-                    {
-                        bbit = 2 * ncnt + 2 * j + 1;
-                        bks = (size_t)i * K + bbit;
-                    }
+                    if (kLights && (fl & F_NMAP) && shadowed) bbit = 2 * ncnt + 2 * j + 1;
+                    const size_t bks = nee_at(R, bbit, i), bh = nee_at(R, bbit >> 1, i);
                     if (mask & (1ull << bbit))
                     {
-                        int4 r = R.nee_res[bks];
-                        float4 nb = R.nee_b[bks];
-                        int Lid = (int)nb.z;
+                        int4 r = R.nee_res[bh];
+                        float2 nb = R.nee_b[bh];
+                        int Lid = (int)nb.y;
                         if (r.x >= 0)
                         {
                             // shadowhit.bundle->GetAreaLight() == &light (ditracer.cpp:202); quirk-free:
@@ -692,8 +703,9 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
                                 Mat lm;
                                 tri_verts(S, r.x, p1, p2, p3, n1, n2, n3, lm);
                                 Frame hh = fill_hit(p1, p2, p3, n1, n2, n3, __int_as_float(r.z), __int_as_float(r.w));
-                                f3 wi = ld3(R.nee_wi[bks]);
-                                f3 d = hh.p - ps;
+                                const float4 wi4 = R.nee_wi[bks];
+                                f3 wi = ld3(wi4);
+                                f3 d = hh.p - ld3(R.ray_o[i]);
                                 f3 le = mk(0.f, 0.f, 0.f);
                                 if (dot(hh.n, -wi) > 0.f)
                                 {
@@ -704,7 +716,7 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
                                 if (sqnorm(le) > 0.f)
                                 {
                                     float4 na = R.nee_a[bks];
-                                    local = local + le * ld3(na) * na.w * nb.x * nb.y;
+                                    local = local + le * ld3(na) * na.w * wi4.w * nb.x;
                                 }
                             }
                         }
@@ -712,11 +724,12 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
                         {
                             // the ray left the scene: the light's GetLe, nonzero for environment
                             // lights (ditracer.cpp:218-222)
-                            f3 le = other_light_le(S, S.lights[Lid], ld3(R.nee_wi[bks]));
+                            const float4 wi4 = R.nee_wi[bks];
+                            f3 le = other_light_le(S, S.lights[Lid], ld3(wi4));
                             if (sqnorm(le) > 0.f)
                             {
                                 float4 na = R.nee_a[bks];
-                                local = local + le * ld3(na) * na.w * nb.x * nb.y;
+                                local = local + le * ld3(na) * na.w * wi4.w * nb.x;
                             }
                         }
                     }
@@ -788,18 +801,6 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
                     f3 wo = -ld3(R.ray_d[i]);
                     uint32_t base = meta.x;
                     f3 T = ld3(R.thr[i]);
-                    float ux, uy;
-                    if (b == 0)
-                    {
-                        nee_sample2d(J.brdf_smp, base, KS_BRDF, 0, ux, uy);   // pre-drawn once per path, gitracer.cpp:36-41
-                        meta.z = __float_as_uint(ux);
-                        meta.w = __float_as_uint(uy);
-                    }
-                    else
-                    {
-                        ux = __uint_as_float(meta.z);
-                        uy = __uint_as_float(meta.w);
-                    }
                     if (b == 0 && m.type == 2)
                     {
                         rad = rad + emissive_le(m.c, h.n, wo);   // gitracer.cpp:61-68
@@ -840,7 +841,7 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
                                 float lx, ly, bx, by;
                                 nee_sample2d(J.light_smp, base, KS_LIGHT, lc, lx, ly);
                                 nee_sample2d(J.brdf_smp, base, KS_BRDF, bc, bx, by);
-                                size_t ks = (size_t)i * K + 2 * j;
+                                const size_t ks = nee_at(R, 2 * j, i);
                                 // light sample + shadow ray
                                 f3 ld;
                                 float lpdf = 0.f, cosl = 0.f;
@@ -908,10 +909,10 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
                                         if (spec || (nq ? lp > 0.f || !area : !(lp < kMinPdf)))
                                         {
                                             float w = spec || (nq && !(lp > 0.f)) ? 1.f : power_heuristic(bpdf, lp);
-                                            const size_t kb = (size_t)i * K + bit;
+                                            const size_t kb = nee_at(R, bit, i);
                                             R.nee_a[kb] = st3(fb, fabsf(dot(hs.n, wi)));
-                                            R.nee_b[kb] = make_float4(nq ? w * pickw : w, 1.f / bpdf, (float)Lid, 0.f);
-                                            R.nee_wi[kb] = st3(wi, 10000000.f);
+                                            R.nee_b[nee_at(R, bit >> 1, i)] = make_float2(1.f / bpdf, (float)Lid);
+                                            R.nee_wi[kb] = st3(wi, nq ? w * pickw : w);
                                             emit_mask |= 1ull << bit;
                                         }
                                     }
@@ -940,7 +941,8 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
                             }
                             R.thr_nee[i] = st3(T, 0.f);
                             R.ray_o[i] = st3(h.p, 0.f);
-                            R.nee_mask[i] = emit_mask;
+                            meta.z = (uint32_t)emit_mask;
+                            meta.w = (uint32_t)(emit_mask >> 32);
                             if (emit_mask) fl |= F_NEE;
                             if (emit_mask && nmref) fl |= F_NMAP;
                             ncnt = jn;
@@ -1013,6 +1015,10 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
                             }
                             else
                             {
+                                // the path's one BSDF sample (pre-drawn before the bounce loop,
+                                // gitracer.cpp:36-41), drawn again from its counter
+                                float ux, uy;
+                                nee_sample2d(J.brdf_smp, base, KS_BRDF, 0, ux, uy);
                                 f = kLights ? mat_sample_x(S.mats, tx, m, h, ux, uy, wo, wi, pdf, type, rs)
                                             : mat_sample(m, h, ux, uy, wo, wi, pdf, type);
                                 stop = sqnorm(f) == 0.f || pdf < kMinPdf;
@@ -1190,21 +1196,21 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
             const unsigned long long m = __ballot(mine);
             if (mine)
             {
-                size_t ks = (size_t)i * K + k;
-                float4 wd = R.nee_wi[ks];
+                const uint32_t ks = i << R.Kshift | (uint32_t)k;
+                float4 wd = R.nee_wi[nee_at(R, k, i)];
                 if (k & 1)
                 {
                     const uint32_t cp = cbase + cofs + (uint32_t)__popcll(m & below);
                     R.qc_o[buf][cp] = st3(org, 0.01f);
-                    R.qc_d[buf][cp] = wd;
-                    R.qc_own[buf][cp] = (int)((Q_NEE_CLOSEST << 29) | (uint32_t)ks);
+                    R.qc_d[buf][cp] = st3(ld3(wd), 10000000.f);
+                    R.qc_own[buf][cp] = (int)((Q_NEE_CLOSEST << 29) | ks);
                 }
                 else
                 {
                     const uint32_t ap = abase + aofs + (uint32_t)__popcll(m & below);
                     R.qa_o[buf][ap] = st3(org, 0.01f);
                     R.qa_d[buf][ap] = wd;
-                    R.qa_own[buf][ap] = (int)((Q_NEE_ANY << 29) | (uint32_t)ks);
+                    R.qa_own[buf][ap] = (int)((Q_NEE_ANY << 29) | ks);
                 }
             }
             if (k & 1) cofs += (uint32_t)__popcll(m);
@@ -1429,14 +1435,14 @@ static bsh_status ensure_work(RenderWork& w, size_t P, int K, int nlmax)
     BSH_HIP(w.out.alloc(P));
     BSH_HIP(w.hit.alloc(P));
     BSH_HIP(w.meta.alloc(P));
-    BSH_HIP(w.nee_mask.alloc(P));
     BSH_HIP(w.alive[0].alloc(P));
     BSH_HIP(w.alive[1].alloc(P));
     size_t slots = P * (size_t)K;
     BSH_HIP(w.nee_a.alloc(slots));
-    BSH_HIP(w.nee_b.alloc(slots));
     BSH_HIP(w.nee_wi.alloc(slots));
-    BSH_HIP(w.nee_res.alloc(slots));
+    BSH_HIP(w.nee_b.alloc(slots / 2));
+    BSH_HIP(w.nee_res.alloc(slots / 2));
+    BSH_HIP(w.nee_occ.alloc(slots / 2));
     size_t qc = P * (size_t)(1 + nlmax), qa = P * (size_t)std::max(nlmax, 1);
     for (int k = 0; k < 2; ++k)
     {
@@ -1959,8 +1965,10 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
         R.Kshift = Kshift;
         R.ray_o = lw.ray_o.p; R.ray_d = lw.ray_d.p; R.thr = lw.thr.p; R.thr_nee = lw.thr_nee.p; R.rad = lw.rad.p;
         R.out = lw.out.p;
-        R.hit = lw.hit.p; R.meta = lw.meta.p; R.nee_mask = lw.nee_mask.p;
+        R.hit = lw.hit.p; R.meta = lw.meta.p;
+        R.nee_stride = (uint32_t)P;
         R.nee_a = lw.nee_a.p; R.nee_b = lw.nee_b.p; R.nee_wi = lw.nee_wi.p; R.nee_res = lw.nee_res.p;
+        R.nee_occ = lw.nee_occ.p;
         for (int k = 0; k < 2; ++k)
         {
             R.qc_o[k] = lw.qc_o[k].p; R.qc_d[k] = lw.qc_d[k].p; R.qc_own[k] = lw.qc_own[k].p;
