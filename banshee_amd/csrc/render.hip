@@ -75,6 +75,10 @@ constexpr int kTraceResidentBlocks = 8, kTraceResidentMulti = 7;
 // plain variant to 5 or 6 waves (96 or 80 VGPRs, 24 or 50 of them spilled) made the 1080p
 // terrain frame 1.1 and 1.5 % slower.
 constexpr int kShadeWavesPerSimd = 4;
+// The kLights variants keep 168 VGPRs (3 waves per SIMD): around their out-of-line material calls a
+// lane spills 304 B instead of 448, and the launches are bound by memory traffic, scratch included
+// (637x361 9-sample frame of mapped materials 3672 us with 4 waves, 3567 with 3, 3563 with 2).
+constexpr int kShadeWavesLights = 3;
 // Statistics buffer: 4 counters, then the guided-row partials, kRowStride apart (128 B), then per
 // bounce launch b: closest rays, any-hit rays, and in counting mode node visits and triangle tests
 // of the closest and of the any-hit rays (kLaunchStat counters each).
@@ -635,7 +639,7 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
 // lights and the materials beyond Lambert, Microfacet and Emissive (material_dev.h), kept out
 // of the other variants' registers.
 template <bool kFull, bool kOne, bool kLights = false>
-__global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev R, int b, int Lout)
+__global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPerSimd) void k_shade(RenderDev R, int b, int Lout)
 {
     // Bounce 0 shades every path of the chunk; a later bounce only the paths the previous
     // shade left live, in the order it listed them (its wave order, so neighbouring paths
@@ -924,27 +928,20 @@ __global__ __launch_bounds__(kBlock, kShadeWavesPerSimd) void k_shade(RenderDev 
                                         }
                                     }
                                 };
-                                if (nmref)
+                                // Sample of a normal-mapped vertex maps the normal as the light branch
+                                // left it: twice where the light sample was unoccluded (Evaluate ran),
+                                // else once. The shadow ray decides later, so both rays are traced.
+                                const bool both = nmref && ((emit_mask >> (2 * j)) & 1ull);
+                                Frame hs = h;
+                                if (nmref) hs.n = both ? nB : nA;
+                                int bit = 2 * j + 1;
+                                for (int v = both ? 1 : 0;; --v)
                                 {
-                                    // Sample maps the normal as the light branch left it: twice where
-                                    // the light sample was unoccluded (Evaluate ran), else once. The
-                                    // shadow ray decides later, so both rays are traced.
-                                    Frame hs = h;
-                                    if ((emit_mask >> (2 * j)) & 1ull)
-                                    {
-                                        hs.n = nB;
-                                        bsdf_nee(hs, 2 * j + 1);
-                                        hs.n = nA;
-                                        bsdf_nee(hs, 2 * jn + 2 * j + 1);
-                                    }
-                                    else
-                                    {
-                                        hs.n = nA;
-                                        bsdf_nee(hs, 2 * j + 1);
-                                    }
+                                    bsdf_nee(hs, bit);
+                                    if (!kLights || v == 0) break;
+                                    hs.n = nA;
+                                    bit = 2 * jn + 2 * j + 1;
                                 }
-                                else
-                                    bsdf_nee(h, 2 * j + 1);
                             }
                             R.thr_nee[i] = st3(T, 0.f);
                             R.ray_o[i] = st3(h.p, 0.f);
