@@ -394,13 +394,25 @@ __global__ __launch_bounds__(kWsumBlock) void k_guide_wsum_final(const float* pa
 // depend on scheduling.
 constexpr int kTrWaves = 8;                                    // waves per block, 16 rows each
 constexpr int kTrRows = 16 * kTrWaves;                         // rows per round
-constexpr int kRp = kTrRows + kPad;                            // staging pitch (halves) per feature
-constexpr int kStIn = 0;                                       // a layer's inputs^T: up to 96 features
-constexpr int kStG = kStIn + kGIn * kRp;                       // its output gradients^T: up to 64
-constexpr int kStLayer = kStG + kGHid * kRp;                   // one staged layer
-constexpr int kStTotal = 2 * kStLayer;                         // two layers at a time
+// Staging areas, row-major: a row of the round per LDS row of up to 64 (or 96) features, with a
+// pitch of 36 (52) banks: the 16 rows x 4 feature groups of a transposed read, and the 16 rows of a
+// write, then spread over all banks. Two layers at a time; only the first area takes layer 1.
+constexpr int kPH = kGHid + kPad, kPI = kGIn + kPad;           // pitches (halves)
+constexpr int kStAIn = 0, kStAG = kStAIn + kTrRows * kPI;      // first area: inputs, output gradients
+constexpr int kStBIn = kStAG + kTrRows * kPH, kStBG = kStBIn + kTrRows * kPH;   // second area
+constexpr int kStTotal = kStBG + kTrRows * kPH;
 constexpr int kPartStride = kGParams + 4;                      // a block's partial sums, then its loss
-static_assert((kRp * 2) % 16 == 0, "16-byte aligned feature rows");
+static_assert((kPH * 2) % 16 == 0 && (kPI * 2) % 16 == 0, "16-byte aligned rows");
+
+// A 16 x 16 tile of halves read transposed from LDS (ds_read_b64_tr_b16): the 16 lanes of group
+// q = lane / 16 name 4 rows of 4 x 4 consecutive halves, lane r those of row r / 4, columns 4 (r % 4) on,
+// and lane r receives column r of the 4 rows.
+typedef short s4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ h4 read_tr(const _Float16* p)
+{
+    typedef __attribute__((address_space(3))) s4v ls4;
+    return __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls4*)p));
+}
 
 // ReLU derivative bits of a layer's four fragments: bit 4 j + i = (h[j][i] > 0).
 __device__ __forceinline__ uint32_t relu_bits(const h4 (&h)[kGHid / 16])
@@ -440,9 +452,9 @@ __device__ __forceinline__ void dense1(const h4 (&x)[K / 16], const _Float16* Wt
     for (int mt = 0; mt < N / 16; ++mt) y[mt] = relu_h4(acc[mt]);
 }
 
-// dH^T = W dOut^T masked by the ReLU bits, with A[m = in][k = out] fragments of W^T read from the
-// forward LDS image (out-major rows, perm32 columns): four rows apart. Out-blocks outer, four
-// independent accumulators.
+// dH^T = W dOut^T masked by the ReLU bits, with A[m = in][k = out] fragments of W^T read transposed
+// from the forward LDS image (out-major rows, perm32 columns, which keep runs of 4 together).
+// Out-blocks outer, four independent accumulators.
 template <int NOUT, int NIN>
 __device__ __forceinline__ void bwd_t(const _Float16* Wt, int ws, const h4 (&dout)[NOUT / 16], uint32_t mask,
                                       h4 (&dh)[NIN / 16], int r, int q)
@@ -456,8 +468,7 @@ __device__ __forceinline__ void bwd_t(const _Float16* Wt, int ws, const h4 (&dou
         h4 a[NIN / 16];
 #pragma unroll
         for (int nt = 0; nt < NIN / 16; ++nt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[nt][i] = Wt[(16 * ks + 4 * q + i) * ws + perm32(16 * nt + r)];
+            a[nt] = read_tr(&Wt[(16 * ks + 4 * q + (r >> 2)) * ws + perm32(16 * nt) + 8 * (r & 3)]);
 #pragma unroll
         for (int nt = 0; nt < NIN / 16; ++nt) acc[nt] = mfma16(a[nt], dout[ks], acc[nt]);
     }
@@ -467,14 +478,12 @@ __device__ __forceinline__ void bwd_t(const _Float16* Wt, int ws, const h4 (&dou
         for (int i = 0; i < 4; ++i) dh[nt][i] = (mask >> (4 * nt + i)) & 1u ? (_Float16)acc[nt][i] : (_Float16)0.f;
 }
 
-// Feature-major staging of the lane's fragments: T[feature][lr].
-template <int N>
+// Row-major staging of the lane's fragments: T[lr][feature], one 8-byte write per fragment.
+template <int N, int kPitch>
 __device__ __forceinline__ void stage_t(_Float16* T, int lr, const h4 (&v)[N / 16], int q)
 {
 #pragma unroll
-    for (int j = 0; j < N / 16; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) T[(16 * j + 4 * q + i) * kRp + lr] = v[j][i];
+    for (int j = 0; j < N / 16; ++j) *reinterpret_cast<h4*>(&T[lr * kPitch + 16 * j + 4 * q]) = v[j];
 }
 
 // One wave's 16 rows (raw inputs a, c and record (dir, weight) d already loaded): the forward
@@ -595,9 +604,17 @@ __device__ __forceinline__ float train_forward(const _Float16* lw, const float* 
 // One layer's weight-gradient tiles of a wave over the round's staged rows: acc[A0 + t] +=
 // In[row][16 (ib0 + t ibstep) + in]^T G[row][16 ob + out] for t < NT (when `tiles`), and with
 // `bias` acc[B0] += sum_rows G[row][16 ob + out] in every row (a product with a ones operand).
-// A[m = in][k = row] and B[k = row][n = out] are 8 consecutive rows of one feature per lane.
+// A[m = in][k = row] and B[k = row][n = out] are 8 consecutive rows of one feature per lane: two
+// transposed reads of 4.
 constexpr int kAccTiles = 16;
-template <int NT, int A0, int B0>
+template <int kPitch>
+__device__ __forceinline__ h8 read_col8(const _Float16* T, int block, int g, int r, int q)
+{
+    const _Float16* p = &T[(32 * g + 8 * q + (r >> 2)) * kPitch + 16 * block + 4 * (r & 3)];
+    return cat8(read_tr(p), read_tr(p + 4 * kPitch));
+}
+
+template <int NT, int A0, int B0, int kPitchIn>
 __device__ __forceinline__ void wgrad_layer(const _Float16* In, const _Float16* G, int ib0, int ibstep, int ob,
                                             bool tiles, bool bias, f4v (&acc)[kAccTiles], int r, int q)
 {
@@ -606,14 +623,14 @@ __device__ __forceinline__ void wgrad_layer(const _Float16* In, const _Float16* 
 #pragma unroll
     for (int g = 0; g < kTrRows / 32; ++g)
     {
-        const h8 b = *reinterpret_cast<const h8*>(&G[(16 * ob + r) * kRp + 32 * g + 8 * q]);
+        const h8 b = read_col8<kPH>(G, ob, g, r, q);
         if (bias) acc[B0] = mfma32(ones, b, acc[B0]);
         if (tiles)
         {
             h8 a[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t)
-                a[t] = *reinterpret_cast<const h8*>(&In[(16 * (ib0 + t * ibstep) + r) * kRp + 32 * g + 8 * q]);
+                a[t] = read_col8<kPitchIn>(In, ib0 + t * ibstep, g, r, q);
 #pragma unroll
             for (int t = 0; t < NT; ++t) acc[A0 + t] = mfma32(a[t], b, acc[A0 + t]);
         }
@@ -659,8 +676,7 @@ __global__ __launch_bounds__(64 * kTrWaves, 1) void k_guide_train_fused(GuideNet
     float loss = 0.f;
     const uint32_t rounds = (nrows + kTrRows - 1) / kTrRows;
     const int lr = 16 * wave + r;
-    _Float16* sA = st;
-    _Float16* sB = st + kStLayer;
+    _Float16 *sAi = st + kStAIn, *sAg = st + kStAG, *sBi = st + kStBIn, *sBg = st + kStBG;
     float* O = ox + wave * 16 * kGOut;
     // the lane's record of the next round, loaded during the current one
     float4 na = make_float4(0.f, 0.f, 0.f, 0.f), nc = na, nd = na;
@@ -689,10 +705,10 @@ __global__ __launch_bounds__(64 * kTrWaves, 1) void k_guide_train_fused(GuideNet
         // the previous round's last weight gradients have read the staging area
         __syncthreads();
         // layers 5 and 4
-        stage_t<kGHid>(sA + kStIn, lr, hh, q);
-        stage_t<kGOut>(sA + kStG, lr, dy, q);
-        stage_t<kGHid>(sB + kStIn, lr, h3, q);
-        stage_t<kGHid>(sB + kStG, lr, g4, q);
+        stage_t<kGHid, kPH>(sAi, lr, hh, q);
+        stage_t<kGOut, kPH>(sAg, lr, dy, q);
+        stage_t<kGHid, kPH>(sBi, lr, h3, q);
+        stage_t<kGHid, kPH>(sBg, lr, g4, q);
         bwd_t<kGHid, kGHid>(W + kLF4, kLHS, g4, m3, g3, r, q);
         // the next round's record, issued here where fewer activations are live
         if (rd + gridDim.x < rounds && nrow < nrows)
@@ -702,27 +718,27 @@ __global__ __launch_bounds__(64 * kTrWaves, 1) void k_guide_train_fused(GuideNet
             nd = rec[(size_t)srow * nrow + 2];
         }
         __syncthreads();
-        wgrad_layer<2, 13, 15>(sA + kStIn, sA + kStG, ib5, 2, ob5, tiles5, bias5, acc, r, q);
-        wgrad_layer<2, 10, 12>(sB + kStIn, sB + kStG, ib, 2, ob, true, bias4, acc, r, q);
+        wgrad_layer<2, 13, 15, kPH>(sAi, sAg, ib5, 2, ob5, tiles5, bias5, acc, r, q);
+        wgrad_layer<2, 10, 12, kPH>(sBi, sBg, ib, 2, ob, true, bias4, acc, r, q);
         // dH2 while the other waves finish reading layers 5 and 4
         bwd_t<kGHid, kGHid>(W + kLF3, kLHS, g3, relu_bits(h2), g2, r, q);
         const uint32_t m1 = relu_bits(h1);
         __syncthreads();
         // layers 3 and 2
-        stage_t<kGHid>(sA + kStIn, lr, h2, q);
-        stage_t<kGHid>(sA + kStG, lr, g3, q);
-        stage_t<kGHid>(sB + kStIn, lr, h1, q);
-        stage_t<kGHid>(sB + kStG, lr, g2, q);
+        stage_t<kGHid, kPH>(sAi, lr, h2, q);
+        stage_t<kGHid, kPH>(sAg, lr, g3, q);
+        stage_t<kGHid, kPH>(sBi, lr, h1, q);
+        stage_t<kGHid, kPH>(sBg, lr, g2, q);
         bwd_t<kGHid, kGHid>(W + kLF2, kLHS, g2, m1, g1, r, q);
         __syncthreads();
-        wgrad_layer<2, 7, 9>(sA + kStIn, sA + kStG, ib, 2, ob, true, bias4, acc, r, q);
-        wgrad_layer<2, 4, 6>(sB + kStIn, sB + kStG, ib, 2, ob, true, bias4, acc, r, q);
+        wgrad_layer<2, 7, 9, kPH>(sAi, sAg, ib, 2, ob, true, bias4, acc, r, q);
+        wgrad_layer<2, 4, 6, kPH>(sBi, sBg, ib, 2, ob, true, bias4, acc, r, q);
         __syncthreads();
         // layer 1
-        stage_t<kGIn>(sA + kStIn, lr, x, q);
-        stage_t<kGHid>(sA + kStG, lr, g1, q);
+        stage_t<kGIn, kPI>(sAi, lr, x, q);
+        stage_t<kGHid, kPH>(sAg, lr, g1, q);
         __syncthreads();
-        wgrad_layer<3, 0, 3>(sA + kStIn, sA + kStG, ib, 2, ob, true, bias4, acc, r, q);
+        wgrad_layer<3, 0, 3, kPI>(sAi, sAg, ib, 2, ob, true, bias4, acc, r, q);
     }
     float* P = part + (size_t)blockIdx.x * kPartStride;
     wgrad_store<3, 0, 3>(P, kGW1, kGB1, kGHid, ib, 2, ob, true, bias4, acc, r, q);
