@@ -56,50 +56,56 @@ __host__ __device__ constexpr int perm32(int k)
 {
     return (k & ~31) | (((k >> 2) & 3) << 3) | (((k >> 4) & 1) << 2) | (k & 3);
 }
-constexpr int kF1 = 0;                                             // 64 rows x 96
-constexpr int kF2 = kF1 + kGHid * kGIn;                            // 64 x 64
-constexpr int kF3 = kF2 + kGHid * kGHid;
-constexpr int kF4 = kF3 + kGHid * kGHid;
-constexpr int kF5 = kF4 + kGHid * kGHid;                           // 48 x 64
-constexpr int kFTotal = kF5 + kGOut * kGHid;
-// ---- backward layout (in-major rows W[n_in][k_out]) for layers 5..2 ----
-constexpr int kB5 = 0;                                             // 64 rows x 48
-constexpr int kB4 = kB5 + kGHid * kGOut;                           // 64 x 64
-constexpr int kB3 = kB4 + kGHid * kGHid;
-constexpr int kB2 = kB3 + kGHid * kGHid;
-constexpr int kBTotal = kB2 + kGHid * kGHid;
 constexpr int kBiasTotal = 4 * kGHid + kGOut;
-// LDS image of the forward weights (padded rows)
+// LDS image of the forward weights (padded rows), then b1..b5
 constexpr int kLF1 = 0, kLF2 = kLF1 + kGHid * kL1S, kLF3 = kLF2 + kGHid * kLHS, kLF4 = kLF3 + kGHid * kLHS,
               kLF5 = kLF4 + kGHid * kLHS, kLFTotal = kLF5 + kGOut * kLHS;
+constexpr int kImgUnits = (kLFTotal * 2 + kBiasTotal * 4) / 16;   // 16-byte units
+static_assert(kLFTotal % 8 == 0 && kBiasTotal % 4 == 0, "whole 16-byte units");
 
+// The device copy of the weights is that image, so a kernel's start is a straight copy into LDS,
+// its loads all in flight together. (Unpadded rows, padded and permuted by each block 8 bytes at a
+// time in a loop of 23 dependent rounds: the fused training step 88.5 us on 2^18 records against
+// 86.7, inference on 2^20 rows 86.9 us against 81.3.)
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 struct GuideNet
 {
-    const _Float16* wf;   // forward FP16 weights (kFTotal)
-    const _Float16* wb;   // backward FP16 weights (kBTotal)
-    const float* bias;    // b1..b5 (kBiasTotal)
+    const u4v* img;
 };
 
-__device__ __forceinline__ void load_fwd_weights(const GuideNet& g, _Float16* lw, float* lb)
+// Where parameter t lives in the image: the half index of a weight (bias -1), or its bias index.
+__device__ __forceinline__ int guide_image_at(int t, int& bias)
 {
-    // unpadded global rows -> padded, column-permuted LDS rows, 4 halves at a time (perm32
-    // keeps runs of 4 consecutive features together)
-    const h4* src = reinterpret_cast<const h4*>(g.wf);
-    for (int u = threadIdx.x; u < kFTotal / 4; u += blockDim.x)
+    bias = -1;
+    if (t < kGB1) return kLF1 + t % kGHid * kL1S + perm32(t / kGHid);
+    const int w[4] = {kGW2, kGW3, kGW4, kGW5}, l[4] = {kLF2, kLF3, kLF4, kLF5};
+    if (t < kGW2) { bias = t - kGB1; return 0; }
+    for (int k = 0; k < 4; ++k)
     {
-        const int t = 4 * u;
-        int dst;
-        if (t < kF2) { int n = t / kGIn, k = t % kGIn; dst = kLF1 + n * kL1S + perm32(k); }
-        else if (t < kF5)
-        {
-            int v = (t - kF2), l = v / (kGHid * kGHid), r = v % (kGHid * kGHid);
-            int n = r / kGHid, k = r % kGHid;
-            dst = kLF2 + l * kGHid * kLHS + n * kLHS + perm32(k);
-        }
-        else { int v = t - kF5; int n = v / kGHid, k = v % kGHid; dst = kLF5 + n * kLHS + perm32(k); }
-        *reinterpret_cast<h4*>(&lw[dst]) = src[u];
+        const int n = k < 3 ? kGHid : kGOut, u = t - w[k];
+        if (u < kGHid * n) return l[k] + u % n * kLHS + perm32(u / n);
+        if (u < kGHid * n + n) { bias = (k + 1) * kGHid + u - kGHid * n; return 0; }
     }
-    for (int t = threadIdx.x; t < kBiasTotal; t += blockDim.x) lb[t] = g.bias[t];
+    return 0;
+}
+
+// Copies the image into LDS (kThreads threads; img: kImgUnits units).
+template <int kThreads>
+__device__ __forceinline__ void load_image(const GuideNet& g, u4v* img)
+{
+    constexpr int kPer = (kImgUnits + kThreads - 1) / kThreads;
+    u4v v[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+    {
+        v[k] = g.img[min((int)threadIdx.x + k * kThreads, kImgUnits - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+    {
+        const int u = threadIdx.x + k * kThreads;
+        if (u < kImgUnits) img[u] = v[k];
+    }
 }
 
 // Encoded input of one row for the lane holding k-positions 4q..4q+3 of every 16-feature
@@ -199,10 +205,11 @@ __global__ __launch_bounds__(64 * kFwdWaves) void k_guide_forward(GuideNet g, co
 {
     constexpr int kGroup = 16 * kFwdTiles;
     static_assert(kGuideSeg % kGroup == 0, "tile groups must not straddle segments");
-    __shared__ __align__(16) _Float16 lw[kLFTotal];
-    __shared__ __align__(16) float lb[kBiasTotal];
-    load_fwd_weights(g, lw, lb);
+    __shared__ u4v img[kImgUnits];
+    load_image<64 * kFwdWaves>(g, img);
     __syncthreads();
+    const _Float16* lw = reinterpret_cast<const _Float16*>(img);
+    const float* lb = reinterpret_cast<const float*>(img + kLFTotal / 8);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, q = lane >> 4;
     const uint32_t ngroups = (nrows + kGroup - 1) / kGroup;
@@ -354,9 +361,16 @@ __device__ __forceinline__ float block_sum(float s, float* red)
     return red[0];
 }
 
-__global__ __launch_bounds__(kWsumBlock) void k_guide_wsum(const float4* rec, int srow, uint32_t nrows, float* part)
+// blockIdx.y: the batch, which starts batch records into `rec` and takes every (srow / 3)-th of them
+// (up to most, of n records in all).
+__global__ __launch_bounds__(kWsumBlock) void k_guide_wsum(const float4* rec, int srow, size_t n, uint32_t most,
+                                                          float* part)
 {
     __shared__ float red[kWsumBlock];
+    const size_t stride = srow / 3, left = (n - blockIdx.y + stride - 1) / stride;
+    const uint32_t nrows = left < most ? (uint32_t)left : most;
+    rec += 3 * (size_t)blockIdx.y;
+    part += blockIdx.y * kWsumParts;
     const uint32_t per = (nrows + kWsumParts - 1) / kWsumParts;
     const uint32_t r0 = blockIdx.x * per, r1 = min(r0 + per, nrows);
     float s = 0.f;
@@ -369,9 +383,10 @@ __global__ __launch_bounds__(kWsumBlock) void k_guide_wsum_final(const float* pa
 {
     __shared__ float red[kWsumBlock];
     float s = 0.f;
+    part += blockIdx.x * kWsumParts;
     for (int k = threadIdx.x; k < kWsumParts; k += kWsumBlock) s += part[k];
     float t = block_sum(s, red);
-    if (threadIdx.x == 0) wsum[0] = t;
+    if (threadIdx.x == 0) wsum[blockIdx.x] = t;
 }
 
 // ---- fused training step ----
@@ -390,7 +405,7 @@ __global__ __launch_bounds__(kWsumBlock) void k_guide_wsum_final(const float* pa
 // a staging, dH2 after a pair's weight gradients, and each is computed as late as its staging
 // allows, which keeps the kernel inside 256 VGPRs without spills. The tiles stay in registers over all the block's
 // rounds (bias gradients as a product with a ones operand); the blocks' partial sums are added
-// in a fixed order by k_guide_reduce_part / k_guide_reduce_train, so a step's result does not
+// in a fixed order by k_guide_update, so a step's result does not
 // depend on scheduling.
 constexpr int kTrWaves = 8;                                    // waves per block, 16 rows each
 constexpr int kTrRows = 16 * kTrWaves;                         // rows per round
@@ -659,13 +674,14 @@ __global__ __launch_bounds__(64 * kTrWaves, 1) void k_guide_train_fused(GuideNet
                                                                         uint32_t nrows, const float* wsum,
                                                                         float* part)
 {
-    __shared__ __align__(16) _Float16 lw[kLFTotal];
-    __shared__ __align__(16) float lb[kBiasTotal];
+    __shared__ u4v img[kImgUnits];
     __shared__ __align__(16) _Float16 st[kStTotal];
     __shared__ __align__(16) float ox[kTrWaves * 16 * kGOut];
     __shared__ float red[kTrWaves];
-    load_fwd_weights(g, lw, lb);
+    load_image<64 * kTrWaves>(g, img);
     __syncthreads();
+    const _Float16* lw = reinterpret_cast<const _Float16*>(img);
+    const float* lb = reinterpret_cast<const float*>(img + kLFTotal / 8);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
     const float scale = (float)nrows / fmaxf(wsum[0], 1e-30f);
     const int ob = wave & 3, ib = wave >> 2, ob5 = wave % 3, ib5 = wave / 3;
@@ -756,43 +772,50 @@ __global__ __launch_bounds__(64 * kTrWaves, 1) void k_guide_train_fused(GuideNet
     }
 }
 
-// Sums the fused kernel's block partials in a fixed order, in two passes so that no thread walks
-// every block: pass 1 (blockIdx.y = group) adds groups of kRedGroup blocks, pass 2 the groups,
-// giving grad = sum / rows and loss = the summed per-row losses.
-constexpr int kRedGroup = 16;
-__global__ void k_guide_reduce_part(const float* part, int nblocks, float* out)
+// Sums the fused kernel's block partials in a fixed order (groups of kRedGroup blocks, then the
+// groups), giving the gradient sum / rows and the summed per-row losses; kAdam: then the Adam step on
+// the FP32 master parameters and the refresh of their FP16 image, else the gradient is stored. A
+// block takes kRedParams parameters, a thread one group of one parameter. Bound by the 22 MB of
+// partials; as three kernels (6.9, 5.4 and 4.7 us on 256 partials) the launches cost more than
+// they read.
+constexpr int kRedGroup = 16, kRedParams = 64, kRedRows = 16, kRedMaxGroups = 32;
+template <bool kAdam>
+__global__ __launch_bounds__(kRedParams * kRedRows) void k_guide_update(const float* __restrict__ part, int nblocks,
+                                                                       float inv_rows, float* grad, float* loss,
+                                                                       float* p, float* m, float* v, float lr,
+                                                                       float b1, float b2, float eps, float c1,
+                                                                       float c2, _Float16* wimg, float* bias)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t > kGParams) return;
-    const int b0 = blockIdx.y * kRedGroup, b1 = min(b0 + kRedGroup, nblocks);
+    __shared__ float gs[kRedMaxGroups][kRedParams];
+    const int col = threadIdx.x % kRedParams, row = threadIdx.x / kRedParams, t = blockIdx.x * kRedParams + col;
+    const int ngroups = (nblocks + kRedGroup - 1) / kRedGroup;
+    for (int g = row; g < ngroups; g += kRedRows)
+    {
+        const int k0 = g * kRedGroup, n = min(kRedGroup, nblocks - k0);
+        float x[kRedGroup];
+#pragma unroll
+        for (int k = 0; k < kRedGroup; ++k) x[k] = (k < n && t <= kGParams) ? part[(size_t)(k0 + k) * kPartStride + t] : 0.f;
+        float s = 0.f;
+#pragma unroll
+        for (int k = 0; k < kRedGroup; ++k)
+            if (k < n) s += x[k];
+        gs[g][col] = s;
+    }
+    __syncthreads();
+    if (row || t > kGParams) return;
     float s = 0.f;
-    for (int b = b0; b < b1; ++b) s += part[(size_t)b * kPartStride + t];
-    out[(size_t)blockIdx.y * kPartStride + t] = s;
-}
-
-__global__ void k_guide_reduce_train(const float* part, int ngroups, float inv_rows, float* grad, float* loss)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t > kGParams) return;
-    float s = 0.f;
-    for (int b = 0; b < ngroups; ++b) s += part[(size_t)b * kPartStride + t];
-    if (t < kGParams) grad[t] = s * inv_rows;
-    else loss[0] = s;
-}
-
-__global__ void k_guide_zero(float* p, int n)
-{
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) p[t] = 0.f;
-}
-
-// Adam on the FP32 master parameters, then refresh the FP16 forward / backward copies.
-__global__ void k_guide_adam(float* p, float* m, float* v, const float* grad, int n, float lr, float b1, float b2,
-                             float eps, float c1, float c2, _Float16* wf, _Float16* wb, float* bias)
-{
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    float g = grad[t];
+    for (int g = 0; g < ngroups; ++g) s += gs[g][col];
+    if (t == kGParams)
+    {
+        loss[0] = s;
+        return;
+    }
+    float g = s * inv_rows;
+    if (!kAdam)
+    {
+        grad[t] = g;
+        return;
+    }
     if (!isfinite(g)) g = 0.f;   // an overflowed entry leaves its parameter as it is
     float mm = b1 * m[t] + (1.f - b1) * g;
     float vv = b2 * v[t] + (1.f - b2) * g * g;
@@ -800,18 +823,16 @@ __global__ void k_guide_adam(float* p, float* m, float* v, const float* grad, in
     v[t] = vv;
     float x = p[t] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
     p[t] = x;
-    // scatter into the FP16 layouts
-    _Float16 hx = (_Float16)x;
-    if (t < kGB1) { int k = t / kGHid, nn = t % kGHid; wf[kF1 + nn * kGIn + k] = hx; }
-    else if (t < kGW2) bias[t - kGB1] = x;
-    else if (t < kGB2) { int u = t - kGW2, k = u / kGHid, nn = u % kGHid; wf[kF2 + nn * kGHid + k] = hx; wb[kB2 + k * kGHid + nn] = hx; }
-    else if (t < kGW3) bias[kGHid + t - kGB2] = x;
-    else if (t < kGB3) { int u = t - kGW3, k = u / kGHid, nn = u % kGHid; wf[kF3 + nn * kGHid + k] = hx; wb[kB3 + k * kGHid + nn] = hx; }
-    else if (t < kGW4) bias[2 * kGHid + t - kGB3] = x;
-    else if (t < kGB4) { int u = t - kGW4, k = u / kGHid, nn = u % kGHid; wf[kF4 + nn * kGHid + k] = hx; wb[kB4 + k * kGHid + nn] = hx; }
-    else if (t < kGW5) bias[3 * kGHid + t - kGB4] = x;
-    else if (t < kGB5) { int u = t - kGW5, k = u / kGOut, nn = u % kGOut; wf[kF5 + nn * kGHid + k] = hx; wb[kB5 + k * kGOut + nn] = hx; }
-    else bias[4 * kGHid + t - kGB5] = x;
+    int bi;
+    const int at = guide_image_at(t, bi);
+    if (bi >= 0) bias[bi] = x;
+    else wimg[at] = (_Float16)x;
+}
+
+__global__ void k_guide_zero(float* p, int n)
+{
+    int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) p[t] = 0.f;
 }
 
 // ---- FP32 mode (verification) ----
@@ -938,10 +959,12 @@ struct bsh_guide
     bsh_context* ctx = nullptr;
     bsh_guide_params prm{};
     std::vector<float> host_params;
-    DevBuf<float> p, m, v, grad, bias, part, part2, loss, wsum;
-    DevBuf<_Float16> wf, wb;
+    DevBuf<float> p, m, v, grad, part, loss, wsum;
+    DevBuf<u4v> img;   // the kernels' weight image
     int step = 0;
-    GuideNet net() const { return GuideNet{wf.p, wb.p, bias.p}; }
+    GuideNet net() const { return GuideNet{img.p}; }
+    _Float16* wimg() const { return reinterpret_cast<_Float16*>(img.p); }
+    float* bias() const { return reinterpret_cast<float*>(img.p + kLFTotal / 8); }
 };
 
 namespace bsh {
@@ -958,36 +981,22 @@ static uint32_t pcg32(uint64_t& st)
 
 static bsh_status upload_params(bsh_guide* g)
 {
-    // fp32 master + derived fp16 copies, built on the host in the same layouts k_guide_adam writes
+    // fp32 master + the derived image, built on the host in the layout k_guide_update writes
     const std::vector<float>& P = g->host_params;
-    std::vector<_Float16> wf(kFTotal), wb(kBTotal);
-    std::vector<float> bias(kBiasTotal);
-    for (int k = 0; k < kGIn; ++k)
-        for (int n = 0; n < kGHid; ++n) wf[kF1 + n * kGIn + k] = (_Float16)P[kGW1 + k * kGHid + n];
-    const int wo[3] = {kGW2, kGW3, kGW4}, fo[3] = {kF2, kF3, kF4}, bo[3] = {kB2, kB3, kB4};
-    for (int l = 0; l < 3; ++l)
-        for (int k = 0; k < kGHid; ++k)
-            for (int n = 0; n < kGHid; ++n)
-            {
-                _Float16 h = (_Float16)P[wo[l] + k * kGHid + n];
-                wf[fo[l] + n * kGHid + k] = h;
-                wb[bo[l] + k * kGHid + n] = h;
-            }
-    for (int k = 0; k < kGHid; ++k)
-        for (int n = 0; n < kGOut; ++n)
-        {
-            _Float16 h = (_Float16)P[kGW5 + k * kGOut + n];
-            wf[kF5 + n * kGHid + k] = h;
-            wb[kB5 + k * kGOut + n] = h;
-        }
-    const int bsrc[5] = {kGB1, kGB2, kGB3, kGB4, kGB5};
-    for (int l = 0; l < 4; ++l)
-        for (int n = 0; n < kGHid; ++n) bias[l * kGHid + n] = P[bsrc[l] + n];
-    for (int n = 0; n < kGOut; ++n) bias[4 * kGHid + n] = P[kGB5 + n];
+    std::vector<u4v> img(kImgUnits, u4v{0u, 0u, 0u, 0u});
+    _Float16* w = reinterpret_cast<_Float16*>(img.data());
+    float* bias = reinterpret_cast<float*>(img.data() + kLFTotal / 8);
+    const int po[5] = {kGW1, kGW2, kGW3, kGW4, kGW5}, lo[5] = {kLF1, kLF2, kLF3, kLF4, kLF5};
+    for (int l = 0; l < 5; ++l)
+    {
+        const int in = l ? kGHid : kGIn, out = l < 4 ? kGHid : kGOut, pitch = l ? kLHS : kL1S;
+        const float* p = P.data() + po[l];
+        for (int k = 0; k < in; ++k)
+            for (int n = 0; n < out; ++n) w[lo[l] + n * pitch + perm32(k)] = (_Float16)p[k * out + n];
+        for (int n = 0; n < out; ++n) bias[l * kGHid + n] = p[in * out + n];
+    }
     BSH_HIP(hipMemcpy(g->p.p, P.data(), kGParams * 4, hipMemcpyHostToDevice));
-    BSH_HIP(hipMemcpy(g->wf.p, wf.data(), kFTotal * 2, hipMemcpyHostToDevice));
-    BSH_HIP(hipMemcpy(g->wb.p, wb.data(), kBTotal * 2, hipMemcpyHostToDevice));
-    BSH_HIP(hipMemcpy(g->bias.p, bias.data(), kBiasTotal * 4, hipMemcpyHostToDevice));
+    BSH_HIP(hipMemcpy(g->img.p, img.data(), kImgUnits * sizeof(u4v), hipMemcpyHostToDevice));
     return BSH_OK;
 }
 
@@ -1017,26 +1026,33 @@ bsh_status guide_forward_rows(bsh_guide* g, const float4* in, const uint32_t* se
     return BSH_OK;
 }
 
-// Forward + backward on `rec` (3 float4 per row); leaves the batch gradient in g->grad
-// and the summed loss (times rows) in g->loss.
-static bsh_status guide_gradients(bsh_guide* g, const float4* rec, int srow, uint32_t n, hipStream_t st)
+// Weight sums of `batches` batches (k_guide_wsum), into g->wsum[0 .. batches).
+constexpr int kMaxSums = 64;
+static bsh_status guide_weight_sums(bsh_guide* g, const float4* rec, int srow, size_t n, uint32_t most, int batches,
+                                    hipStream_t st)
 {
-    const int ncu = g->ctx->num_cus;
-    const uint32_t nb = std::min<uint32_t>((n + kTrRows - 1) / kTrRows, (uint32_t)ncu);
-    const uint32_t ngroups = (nb + kRedGroup - 1) / kRedGroup;
-    if (!g->part.p) BSH_HIP(g->part.alloc((size_t)ncu * kPartStride));
-    if (!g->part2.p) BSH_HIP(g->part2.alloc((size_t)((ncu + kRedGroup - 1) / kRedGroup) * kPartStride));
-    hipLaunchKernelGGL(k_guide_wsum, dim3(kWsumParts), dim3(kWsumBlock), 0, st, rec, srow, n, g->wsum.p + 1);
-    hipLaunchKernelGGL(k_guide_wsum_final, dim3(1), dim3(kWsumBlock), 0, st, g->wsum.p + 1, g->wsum.p);
-    hipLaunchKernelGGL(k_guide_train_fused, dim3(nb), dim3(64 * kTrWaves), 0, st, g->net(), rec, srow, n,
-                       (const float*)g->wsum.p, g->part.p);
-    const dim3 rg((kGParams + 1 + 255) / 256, ngroups);
-    hipLaunchKernelGGL(k_guide_reduce_part, rg, dim3(256), 0, st, (const float*)g->part.p, (int)nb, g->part2.p);
-    hipLaunchKernelGGL(k_guide_reduce_train, dim3(rg.x), dim3(256), 0, st, (const float*)g->part2.p, (int)ngroups,
-                       1.f / (float)n, g->grad.p, g->loss.p);
+    hipLaunchKernelGGL(k_guide_wsum, dim3(kWsumParts, batches), dim3(kWsumBlock), 0, st, rec, srow, n, most,
+                       g->wsum.p + kMaxSums);
+    hipLaunchKernelGGL(k_guide_wsum_final, dim3(batches), dim3(kWsumBlock), 0, st, g->wsum.p + kMaxSums, g->wsum.p);
     BSH_HIP(hipGetLastError());
     return BSH_OK;
 }
+
+// Forward + backward on n rows of `rec` (3 float4 per row) with the weight sum `wsum`: the blocks'
+// partial gradients in g->part. Returns how many blocks in nblocks.
+static bsh_status guide_gradients(bsh_guide* g, const float4* rec, int srow, uint32_t n, const float* wsum, int& nblocks,
+                                  hipStream_t st)
+{
+    const int ncu = std::min(g->ctx->num_cus, kRedGroup * kRedMaxGroups);
+    const uint32_t nb = std::min<uint32_t>((n + kTrRows - 1) / kTrRows, (uint32_t)ncu);
+    if (!g->part.p) BSH_HIP(g->part.alloc((size_t)ncu * kPartStride));
+    hipLaunchKernelGGL(k_guide_train_fused, dim3(nb), dim3(64 * kTrWaves), 0, st, g->net(), rec, srow, n, wsum,
+                       g->part.p);
+    BSH_HIP(hipGetLastError());
+    nblocks = (int)nb;
+    return BSH_OK;
+}
+constexpr int kUpdateBlocks = (kGParams + 1 + kRedParams - 1) / kRedParams;
 
 // FP32 mode: the buffers of one call (features, the four hidden activations, outputs, the
 // output gradient, two ping-pong hidden gradients, the parameter gradient). Allocated per
@@ -1081,9 +1097,9 @@ static bsh_status f32_gradients(bsh_guide* g, const float4* rec, uint32_t n, F32
     BSH_HIP(w.grad.alloc(kGParams));
     hipLaunchKernelGGL(k_guide_zero, dim3(1), dim3(64), 0, st, g->wsum.p, 1);
     hipLaunchKernelGGL(k_guide_zero, dim3(1), dim3(64), 0, st, g->loss.p, 1);
-    hipLaunchKernelGGL(k_guide_wsum, dim3(kWsumParts), dim3(kWsumBlock), 0, st, rec, 3, n, g->wsum.p + 1);
-    hipLaunchKernelGGL(k_guide_wsum_final, dim3(1), dim3(kWsumBlock), 0, st, g->wsum.p + 1, g->wsum.p);
-    bsh_status r = f32_forward(g, rec, 3, n, w, w.out.p, st);
+    bsh_status r = guide_weight_sums(g, rec, 3, n, n, 1, st);
+    if (r != BSH_OK) return r;
+    r = f32_forward(g, rec, 3, n, w, w.out.p, st);
     if (r != BSH_OK) return r;
     hipLaunchKernelGGL(k_guide_loss<float>, dim3((n + 255) / 256), dim3(256), 0, st, (const float*)w.out.p, rec, 3, n,
                        (const float*)g->wsum.p, w.dY.p, g->loss.p);
@@ -1152,11 +1168,9 @@ bsh_status bsh_guide_create(bsh_context* ctx, const bsh_guide_params* prm, bsh_g
         BSH_HIP(g->m.alloc(kGParams));
         BSH_HIP(g->v.alloc(kGParams));
         BSH_HIP(g->grad.alloc(kGParams));
-        BSH_HIP(g->bias.alloc(kBiasTotal));
-        BSH_HIP(g->wf.alloc(kFTotal));
-        BSH_HIP(g->wb.alloc(kBTotal));
+        BSH_HIP(g->img.alloc(kImgUnits));
         BSH_HIP(g->loss.alloc(1));
-        BSH_HIP(g->wsum.alloc(1 + kWsumParts));   // the sum, then the partial sums
+        BSH_HIP(g->wsum.alloc(kMaxSums * (1 + kWsumParts)));   // the sums, then the partial sums
         BSH_HIP(hipMemset(g->m.p, 0, kGParams * 4));
         BSH_HIP(hipMemset(g->v.p, 0, kGParams * 4));
         return BSH_OK;
@@ -1240,8 +1254,17 @@ bsh_status bsh_guide_gradient(bsh_guide* g, const float* records, size_t n, floa
     if (!g || !records || n == 0) return fail(BSH_ERR_INVALID, "bsh_guide_gradient: bad argument");
     if (n >= ((size_t)1 << 30)) return fail(BSH_ERR_UNSUPPORTED, "bsh_guide_gradient: too many rows");
     BSH_HIP(hipSetDevice(g->ctx->device));
-    bsh_status r = guide_gradients(g, reinterpret_cast<const float4*>(records), 3, (uint32_t)n, nullptr);
+    const float4* rec = reinterpret_cast<const float4*>(records);
+    bsh_status r = guide_weight_sums(g, rec, 3, n, (uint32_t)n, 1, nullptr);
     if (r != BSH_OK) return r;
+    int nb = 0;
+    r = guide_gradients(g, rec, 3, (uint32_t)n, g->wsum.p, nb, nullptr);
+    if (r != BSH_OK) return r;
+    hipLaunchKernelGGL(k_guide_update<false>, dim3(kUpdateBlocks), dim3(kRedParams * kRedRows), 0, nullptr,
+                       (const float*)g->part.p, nb, 1.f / (float)n, g->grad.p, g->loss.p, (float*)nullptr,
+                       (float*)nullptr, (float*)nullptr, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, (_Float16*)nullptr,
+                       (float*)nullptr);
+    BSH_HIP(hipGetLastError());
     BSH_HIP(hipDeviceSynchronize());
     if (grad) BSH_HIP(hipMemcpy(grad, g->grad.p, kGParams * 4, hipMemcpyDeviceToHost));
     if (loss)
@@ -1285,17 +1308,19 @@ bsh_status bsh_guide_gradient_fp32(bsh_guide* g, const float* records, size_t n,
     return BSH_OK;
 }
 
-// One Adam step on n records read `stride` records apart.
-static bsh_status train_step(bsh_guide* g, const float* records, size_t stride, size_t n, float* loss,
-                             hipStream_t st)
+// One Adam step on n records read `stride` records apart, whose weight sum is at `wsum`.
+static bsh_status train_step(bsh_guide* g, const float* records, size_t stride, size_t n, const float* wsum,
+                             float* loss, hipStream_t st)
 {
-    bsh_status r = guide_gradients(g, reinterpret_cast<const float4*>(records), (int)(3 * stride), (uint32_t)n, st);
+    int nb = 0;
+    bsh_status r = guide_gradients(g, reinterpret_cast<const float4*>(records), (int)(3 * stride), (uint32_t)n, wsum,
+                                   nb, st);
     if (r != BSH_OK) return r;
     g->step++;
     float c1 = 1.f - std::pow(g->prm.beta1, (float)g->step), c2 = 1.f - std::pow(g->prm.beta2, (float)g->step);
-    hipLaunchKernelGGL(k_guide_adam, dim3((kGParams + 255) / 256), dim3(256), 0, st, g->p.p, g->m.p, g->v.p, g->grad.p,
-                       kGParams, g->prm.lr, g->prm.beta1, g->prm.beta2, g->prm.eps, c1, c2, g->wf.p, g->wb.p,
-                       g->bias.p);
+    hipLaunchKernelGGL(k_guide_update<true>, dim3(kUpdateBlocks), dim3(kRedParams * kRedRows), 0, st,
+                       (const float*)g->part.p, nb, 1.f / (float)n, (float*)nullptr, g->loss.p, g->p.p, g->m.p, g->v.p,
+                       g->prm.lr, g->prm.beta1, g->prm.beta2, g->prm.eps, c1, c2, g->wimg(), g->bias());
     BSH_HIP(hipGetLastError());
     if (loss)
     {
@@ -1313,7 +1338,9 @@ bsh_status bsh_guide_train_step(bsh_guide* g, const float* records, size_t n, fl
     if (n == 0) return BSH_OK;
     if (n >= ((size_t)1 << 30)) return fail(BSH_ERR_UNSUPPORTED, "bsh_guide_train_step: too many rows");
     BSH_HIP(hipSetDevice(g->ctx->device));
-    return train_step(g, records, 1, n, loss, (hipStream_t)stream);
+    bsh_status r = guide_weight_sums(g, reinterpret_cast<const float4*>(records), 3, n, (uint32_t)n, 1, (hipStream_t)stream);
+    if (r != BSH_OK) return r;
+    return train_step(g, records, 1, n, g->wsum.p, loss, (hipStream_t)stream);
 }
 
 bsh_status bsh_guide_train(bsh_guide* g, const float* records, size_t n, int steps, size_t batch, float* loss,
@@ -1328,12 +1355,24 @@ bsh_status bsh_guide_train(bsh_guide* g, const float* records, size_t n, int ste
     // record array (records are in path order, i.e. image order), and successive steps see
     // different records
     const size_t stride = std::max<size_t>(1, n / batch);
+    // the batches' weight sums first, up to kMaxSums of them at a time: a step's batch is its offset's,
+    // so no more than `stride` are distinct, and one launch reads them together
+    size_t sum0 = 0, sums = 0;
     for (int s = 0; s < steps; ++s)
     {
         const size_t off = (size_t)s % stride;
         const size_t rows = std::min(batch, (n - off + stride - 1) / stride);
-        bsh_status r = train_step(g, records + off * 12, stride, rows, s + 1 == steps ? loss : nullptr,
-                                  (hipStream_t)stream);
+        if (off < sum0 || off >= sum0 + sums)
+        {
+            sum0 = off;
+            sums = std::min<size_t>({stride - off, (size_t)kMaxSums, (size_t)(steps - s)});
+            bsh_status r = guide_weight_sums(g, reinterpret_cast<const float4*>(records + off * 12), (int)(3 * stride),
+                                             n - off, (uint32_t)std::min<size_t>(batch, 0xffffffffu), (int)sums,
+                                             (hipStream_t)stream);
+            if (r != BSH_OK) return r;
+        }
+        bsh_status r = train_step(g, records + off * 12, stride, rows, g->wsum.p + (off - sum0),
+                                  s + 1 == steps ? loss : nullptr, (hipStream_t)stream);
         if (r != BSH_OK) return r;
     }
     return BSH_OK;
