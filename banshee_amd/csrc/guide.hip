@@ -396,11 +396,13 @@ __global__ __launch_bounds__(kWsumBlock) void k_guide_wsum_final(const float* pa
 // outputs (4 lanes per row, two lobes each), then the backward pass layer by layer as the
 // transposed products dH^T = W dOut^T masked by H > 0, so every activation and gradient stays in
 // the forward's register layout (lane r + 16 q: row r, features 16 j + 4 q + i). For each layer
-// the waves stage its inputs In_l and output gradients G_l feature-major in LDS (one LDS row per
-// feature, one column per row of the round), compute the next layer's gradient, and after a
-// block barrier add the round's 128 rows to the weight-gradient tiles they own with 16x32
-// products whose operands are 8 rows of one feature, one 16-byte LDS read. Two layers are
-// staged at a time (five layers, six barriers per round; LDS 157 KB). The backward products read
+// the waves stage its inputs In_l and output gradients G_l in LDS (one LDS row per row of the
+// round), compute the next layer's gradient, and after a block barrier add the round's 128 rows
+// to the weight-gradient tiles they own with 16x32 products whose operands are 8 rows of one
+// feature, two transposed LDS reads. Two layers are staged at a time (five layers, six barriers
+// per round; LDS 158 KB). What bounds it is LDS bandwidth: about 19,000 of a round's 25,000 cycles
+// (the weight gradients' transposed reads 7,200, the two passes' weight reads 6,000, staging
+// 2,400, the exchange of the outputs 3,000), the matrix cores busy for a fifth of the time. The backward products read
 // only the weight image, so they fill the waits at the barriers: dH3 and dH1 are computed after
 // a staging, dH2 after a pair's weight gradients, and each is computed as late as its staging
 // allows, which keeps the kernel inside 256 VGPRs without spills. The tiles stay in registers over all the block's
@@ -416,6 +418,10 @@ constexpr int kPH = kGHid + kPad, kPI = kGIn + kPad;           // pitches (halve
 constexpr int kStAIn = 0, kStAG = kStAIn + kTrRows * kPI;      // first area: inputs, output gradients
 constexpr int kStBIn = kStAG + kTrRows * kPH, kStBG = kStBIn + kTrRows * kPH;   // second area
 constexpr int kStTotal = kStBG + kTrRows * kPH;
+// Pitch of the outputs' exchange rows (floats): 52 = -12 mod 64 banks puts the 16 rows' 16-byte writes
+// on 16 different groups of four banks, as it does their 4-byte reads; kGOut itself puts them on four
+// (a write 32 cycles instead of 14). The step on 2^18 records: 86.7 us with 48, 83.6 with 52.
+constexpr int kOP = kGOut + 4;
 constexpr int kPartStride = kGParams + 4;                      // a block's partial sums, then its loss
 static_assert((kPH * 2) % 16 == 0 && (kPI * 2) % 16 == 0, "16-byte aligned rows");
 
@@ -503,7 +509,7 @@ __device__ __forceinline__ void stage_t(_Float16* T, int lr, const h4 (&v)[N / 1
 
 // One wave's 16 rows (raw inputs a, c and record (dir, weight) d already loaded): the forward
 // pass into x and h1..h4, the loss gradient with respect to the outputs into dy (the backward's
-// B fragments). O: the wave's 16 x 48 exchange area. Returns the wave's summed loss (every lane
+// B fragments). O: the wave's exchange area, 16 rows of 48 floats. Returns the wave's summed loss (every lane
 // the same value).
 __device__ __forceinline__ float train_forward(const _Float16* lw, const float* lb, float* O, float4 a, float4 c,
                                                float4 d, bool live, float scale, int r, int q, h4 (&x)[kGIn / 16],
@@ -535,12 +541,12 @@ __device__ __forceinline__ float train_forward(const _Float16* lw, const float* 
         }
 #pragma unroll
         for (int mt = 0; mt < kGOut / 16; ++mt)
-            *reinterpret_cast<float4*>(&O[r * kGOut + mt * 16 + 4 * q]) =
+            *reinterpret_cast<float4*>(&O[r * kOP + mt * 16 + 4 * q]) =
                 make_float4(acc[mt][0], acc[mt][1], acc[mt][2], acc[mt][3]);
     }
     __builtin_amdgcn_wave_barrier();   // the wave's LDS accesses complete in order
     // loss -s log q(w) and its gradient (k_guide_loss's formulas); lane q takes lobes 2q, 2q+1
-    const float* o = O + r * kGOut;
+    const float* o = O + r * kOP;
     float mx = o[0];
 #pragma unroll
     for (int k = 1; k < kGLobes; ++k) mx = fmaxf(mx, o[k]);
@@ -594,7 +600,7 @@ __device__ __forceinline__ float train_forward(const _Float16* lw, const float* 
     float loss = (ok && q == 0) ? -sw * logf(qm) : 0.f;
     __builtin_amdgcn_wave_barrier();   // every output read before the area holds the gradient
     // the row's 48 output gradients as halves over the exchange area, this lane's 12 of them
-    _Float16* Y = reinterpret_cast<_Float16*>(O) + r * kGOut;
+    _Float16* Y = reinterpret_cast<_Float16*>(O + r * kOP);
     Y[2 * q] = (_Float16)gl[0];
     Y[2 * q + 1] = (_Float16)gl[1];
     Y[8 + 6 * q + 0] = (_Float16)gmu[0].x;
@@ -676,7 +682,7 @@ __global__ __launch_bounds__(64 * kTrWaves, 1) void k_guide_train_fused(GuideNet
 {
     __shared__ u4v img[kImgUnits];
     __shared__ __align__(16) _Float16 st[kStTotal];
-    __shared__ __align__(16) float ox[kTrWaves * 16 * kGOut];
+    __shared__ __align__(16) float ox[kTrWaves * 16 * kOP];
     __shared__ float red[kTrWaves];
     load_image<64 * kTrWaves>(g, img);
     __syncthreads();
@@ -693,7 +699,7 @@ __global__ __launch_bounds__(64 * kTrWaves, 1) void k_guide_train_fused(GuideNet
     const uint32_t rounds = (nrows + kTrRows - 1) / kTrRows;
     const int lr = 16 * wave + r;
     _Float16 *sAi = st + kStAIn, *sAg = st + kStAG, *sBi = st + kStBIn, *sBg = st + kStBG;
-    float* O = ox + wave * 16 * kGOut;
+    float* O = ox + wave * 16 * kOP;
     // the lane's record of the next round, loaded during the current one
     float4 na = make_float4(0.f, 0.f, 0.f, 0.f), nc = na, nd = na;
     uint32_t nrow = blockIdx.x * kTrRows + lr;
