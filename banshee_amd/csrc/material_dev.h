@@ -8,6 +8,7 @@
 
 #include "bsh_math.h"
 #include "light_dev.h"
+#include "scene_dev.h"
 
 namespace bsh {
 
@@ -273,9 +274,40 @@ BSH_HD Mat mixed_pick(const float4* mats, const TexCtx& tx, const Mat& m, bool r
     return c;
 }
 
-// Material::Sample of every material type; rs advances for Glass and MixedMaterial.
-static __device__ __noinline__ f3 mat_sample_x(const float4* mats, const TexCtx& tx, const Mat& m, const Frame& h, float ux, float uy, f3 wi, f3& wo, float& pdf,
-                       int& type, RandStream& rs)
+// Material::Sample, Evaluate and GetPdf of every material type are calls: inlined at each of their
+// sites they are 50,000 instructions and spill. Every argument and result is a scalar or a small
+// struct passed in registers (at most 32), and the scene's tables, which only mixtures read, go
+// by the scene's address. By reference, the material, the frame and the results lived in the lanes'
+// scratch memory: the shade launches of a 637 x 361 9-sample pass with mapped materials wrote
+// 4.5 GB in 2.8 ms, most of it scratch; by value 1.8 GB in 1.6 ms.
+
+// The material and the frame's directions from a call's scalar arguments (the position is not used).
+#define BSH_MAT_PARAMS \
+    int mtype, float mcx, float mcy, float mcz, float meta, float malpha, float mx, float my, float nx, float ny, \
+        float nz, float gx, float gy, float gz, float ax, float ay, float az, float bx, float by, float bz
+#define BSH_MAT_ARGS(m, h) \
+    m.type, m.c.x, m.c.y, m.c.z, m.eta, m.alpha, m.x, m.y, h.n.x, h.n.y, h.n.z, h.ng.x, h.ng.y, h.ng.z, h.dpdu.x, \
+        h.dpdu.y, h.dpdu.z, h.dpdv.x, h.dpdv.y, h.dpdv.z
+#define BSH_MAT_LOCALS \
+    const Mat m{mtype, mk(mcx, mcy, mcz), meta, malpha, mx, my}; \
+    const Frame h{mk(0.f, 0.f, 0.f), mk(nx, ny, nz), mk(gx, gy, gz), mk(ax, ay, az), mk(bx, by, bz)};
+
+BSH_HD TexCtx scene_maps(const SceneDev* s, float u, float v)
+{
+    return TexCtx{s->tex, s->tex_desc, s->mat_maps, u, v};
+}
+
+struct MatSample
+{
+    f3 f, wo;
+    float pdf;
+    int type;
+    uint32_t c;   // the rand() stream's counter after the call
+};
+
+// Material::Sample; the stream advances for Glass and MixedMaterial.
+BSH_HD f3 mat_sample_any(const SceneDev* s, float u, float v, const Mat& m, const Frame& h, float ux, float uy, f3 wi,
+                         f3& wo, float& pdf, int& type, RandStream& rs)
 {
     if (m.type <= MAT_EMISSIVE) return mat_sample(m, h, ux, uy, wi, wo, pdf, type);
     if (m.type == MAT_GLASS)
@@ -303,13 +335,13 @@ static __device__ __noinline__ f3 mat_sample_x(const float4* mats, const TexCtx&
     {
         // MixedMaterial::Sample (mixedmaterial.h:57-87)
         int nr, nt;
-        mixed_counts(mats, m, nr, nt);
+        mixed_counts(s->mats, m, nr, nt);
         float reflectance = fresnel_dielectric(1.f, m.eta, dot(h.n, wi));
         float rnd = rs.next_float();
         const bool refl = nt == 0 || rnd < reflectance;
         const int cnt = refl ? nr : nt;
         const int idx = (int)(rs.next_uint() % (uint32_t)cnt);
-        const Mat c = mixed_pick(mats, tx, m, refl, idx);
+        const Mat c = mixed_pick(s->mats, scene_maps(s, u, v), m, refl, idx);
         f3 f = bsdf_sample(c, h, ux, uy, wi, wo, pdf);
         type = bsdf_flags(c.type);
         pdf *= (1.f / (float)cnt);
@@ -319,8 +351,8 @@ static __device__ __noinline__ f3 mat_sample_x(const float4* mats, const TexCtx&
     return bsdf_sample(m, h, ux, uy, wi, wo, pdf);
 }
 
-// Material::Evaluate of every material type (Glass: 0, glass.h:87-90).
-static __device__ __noinline__ f3 mat_eval_x(const float4* mats, const TexCtx& tx, const Mat& m, const Frame& h, f3 wi, f3 wo)
+// Material::Evaluate (Glass: 0, glass.h:87-90).
+BSH_HD f3 mat_eval_any(const SceneDev* s, float u, float v, const Mat& m, const Frame& h, f3 wi, f3 wo)
 {
     if (m.type <= MAT_EMISSIVE) return mat_eval(m, h, wi, wo);
     if (m.type == MAT_GLASS) return mk(0.f, 0.f, 0.f);
@@ -335,8 +367,8 @@ static __device__ __noinline__ f3 mat_eval_x(const float4* mats, const TexCtx& t
         {
             int id = (int)ids[k];
             if (id < 0) continue;
-            Mat c = load_mat(mats, id);
-            apply_maps(tx, id, c);
+            Mat c = load_mat(s->mats, id);
+            apply_maps(scene_maps(s, u, v), id, c);
             if (((bsdf_flags(c.type) & BSDF_REFLECTION) != 0) == refl) f = f + bsdf_eval(c, h, wi, wo);
         }
         return f;
@@ -344,8 +376,8 @@ static __device__ __noinline__ f3 mat_eval_x(const float4* mats, const TexCtx& t
     return bsdf_eval(m, h, wi, wo);
 }
 
-// Material::GetPdf of every material type (Glass: 0, glass.h:82-85).
-static __device__ __noinline__ float mat_pdf_x(const float4* mats, const TexCtx& tx, const Mat& m, const Frame& h, f3 wi, f3 wo)
+// Material::GetPdf (Glass: 0, glass.h:82-85).
+BSH_HD float mat_pdf_any(const SceneDev* s, float u, float v, const Mat& m, const Frame& h, f3 wi, f3 wo)
 {
     if (m.type <= MAT_EMISSIVE) return mat_pdf(m, h, wi, wo);
     if (m.type == MAT_GLASS) return 0.f;
@@ -361,8 +393,8 @@ static __device__ __noinline__ float mat_pdf_x(const float4* mats, const TexCtx&
         {
             int id = (int)ids[k];
             if (id < 0) continue;
-            Mat c = load_mat(mats, id);
-            apply_maps(tx, id, c);
+            Mat c = load_mat(s->mats, id);
+            apply_maps(scene_maps(s, u, v), id, c);
             if (((bsdf_flags(c.type) & BSDF_REFLECTION) != 0) == refl)
             {
                 pdf += bsdf_pdf(c, h, wi, wo);
@@ -374,5 +406,58 @@ static __device__ __noinline__ float mat_pdf_x(const float4* mats, const TexCtx&
     }
     return bsdf_pdf(m, h, wi, wo);
 }
+
+static __device__ __noinline__ MatSample mat_sample_call(const SceneDev* s, float u, float v, BSH_MAT_PARAMS, float ux,
+                                                         float uy, float wix, float wiy, float wiz, uint32_t base,
+                                                         uint32_t c)
+{
+    BSH_MAT_LOCALS
+    RandStream rs{base, c};
+    MatSample r{mk(0.f, 0.f, 0.f), mk(0.f, 0.f, 0.f), 0.f, 0, 0u};
+    r.f = mat_sample_any(s, u, v, m, h, ux, uy, mk(wix, wiy, wiz), r.wo, r.pdf, r.type, rs);
+    r.c = rs.c;
+    return r;
+}
+
+static __device__ __noinline__ f3 mat_eval_call(const SceneDev* s, float u, float v, BSH_MAT_PARAMS, float wix,
+                                                float wiy, float wiz, float wox, float woy, float woz)
+{
+    BSH_MAT_LOCALS
+    return mat_eval_any(s, u, v, m, h, mk(wix, wiy, wiz), mk(wox, woy, woz));
+}
+
+static __device__ __noinline__ float mat_pdf_call(const SceneDev* s, float u, float v, BSH_MAT_PARAMS, float wix,
+                                                  float wiy, float wiz, float wox, float woy, float woz)
+{
+    BSH_MAT_LOCALS
+    return mat_pdf_any(s, u, v, m, h, mk(wix, wiy, wiz), mk(wox, woy, woz));
+}
+
+// s: the scene where it lies in memory (a local copy's address would put the copy in scratch).
+__device__ __forceinline__ f3 mat_sample_x(const SceneDev* s, const TexCtx& tx, const Mat& m, const Frame& h, float ux,
+                                           float uy, f3 wi, f3& wo, float& pdf, int& type, RandStream& rs)
+{
+    const MatSample r =
+        mat_sample_call(s, tx.u, tx.v, BSH_MAT_ARGS(m, h), ux, uy, wi.x, wi.y, wi.z, rs.base, rs.c);
+    wo = r.wo;
+    pdf = r.pdf;
+    type = r.type;
+    rs.c = r.c;
+    return r.f;
+}
+
+__device__ __forceinline__ f3 mat_eval_x(const SceneDev* s, const TexCtx& tx, const Mat& m, const Frame& h, f3 wi, f3 wo)
+{
+    return mat_eval_call(s, tx.u, tx.v, BSH_MAT_ARGS(m, h), wi.x, wi.y, wi.z, wo.x, wo.y, wo.z);
+}
+
+__device__ __forceinline__ float mat_pdf_x(const SceneDev* s, const TexCtx& tx, const Mat& m, const Frame& h, f3 wi,
+                                           f3 wo)
+{
+    return mat_pdf_call(s, tx.u, tx.v, BSH_MAT_ARGS(m, h), wi.x, wi.y, wi.z, wo.x, wo.y, wo.z);
+}
+#undef BSH_MAT_PARAMS
+#undef BSH_MAT_ARGS
+#undef BSH_MAT_LOCALS
 
 }  // namespace bsh

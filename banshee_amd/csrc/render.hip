@@ -75,9 +75,9 @@ constexpr int kTraceResidentBlocks = 8, kTraceResidentMulti = 7;
 // plain variant to 5 or 6 waves (96 or 80 VGPRs, 24 or 50 of them spilled) made the 1080p
 // terrain frame 1.1 and 1.5 % slower.
 constexpr int kShadeWavesPerSimd = 4;
-// The kLights variants keep 168 VGPRs (3 waves per SIMD): around their out-of-line material calls a
-// lane spills 304 B instead of 448, and the launches are bound by memory traffic, scratch included
-// (637x361 9-sample frame of mapped materials 3672 us with 4 waves, 3567 with 3, 3563 with 2).
+// The kLights variants keep 168 VGPRs (3 waves per SIMD), of which a lane spills 48 B around the
+// material calls: a 637x361 9-sample frame of mapped materials 2525 us with 4 waves (208 B), 2340
+// with 3, 2690 with 2 (no spills).
 constexpr int kShadeWavesLights = 3;
 // Statistics buffer: 4 counters, then the guided-row partials, kRowStride apart (128 B), then per
 // bounce launch b: closest rays, any-hit rays, and in counting mode node visits and triangle tests
@@ -871,7 +871,7 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
                                     // for the cosine) and GetPdf maps that copy again (nB)
                                     Frame hE = h;
                                     if (nmref) hE.n = nA;
-                                    f3 f = kLights ? mat_eval_x(S.mats, tx, m, hE, wi, wo) : mat_eval(m, h, wi, wo);
+                                    f3 f = kLights ? mat_eval_x(&J.s, tx, m, hE, wi, wo) : mat_eval(m, h, wi, wo);
                                     float w = 1.f;
                                     if (!singular)
                                     {
@@ -880,7 +880,7 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
                                         // direction from the view, GetPdf(view, light dir)
                                         Frame hP = h;
                                         if (nmref) hP.n = nB;
-                                        float bp = kLights ? (nq ? mat_pdf_x(S.mats, tx, m, h, wo, wi) : mat_pdf_x(S.mats, tx, m, hP, wi, wo))
+                                        float bp = kLights ? (nq ? mat_pdf_x(&J.s, tx, m, h, wo, wi) : mat_pdf_x(&J.s, tx, m, hP, wi, wo))
                                                            : (nq ? mat_pdf(m, h, wo, wi) : mat_pdf(m, h, wi, wo));
                                         // quirk-free: both MIS weights in solid angle (the reference
                                         // weighs an area light's area pdf against the BSDF's solid-angle
@@ -905,7 +905,7 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
                                     float bpdf = 0.f;
                                     int type = 0;
                                     f3 fb = singular ? mk(0.f, 0.f, 0.f)
-                                                     : kLights ? mat_sample_x(S.mats, tx, m, hs, bx, by, wo, wis, bpdf, type, rs)
+                                                     : kLights ? mat_sample_x(&J.s, tx, m, hs, bx, by, wo, wis, bpdf, type, rs)
                                                                : mat_sample(m, hs, bx, by, wo, wis, bpdf, type);
                                     f3 wi = normalize(wis);
                                     if (!singular && sqnorm(fb) > 0.f && (nq ? bpdf > 0.f : bpdf > kMinPdf))
@@ -991,12 +991,12 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
                                 f3 fown = mk(0.f, 0.f, 0.f);
                                 if (own)
                                 {
-                                    fown = mat_sample_x(S.mats, tx, m, h, gx, gy, wo, wi, pdf, type, rs);
+                                    fown = mat_sample_x(&J.s, tx, m, h, gx, gy, wo, wi, pdf, type, rs);
                                     wi = normalize(wi);
                                 }
                                 else if (!guided || usel < alpha)
                                 {
-                                    if (kLights) (void)mat_sample_x(S.mats, tx, m, h, gx, gy, wo, wi, pdf, type, rs);
+                                    if (kLights) (void)mat_sample_x(&J.s, tx, m, h, gx, gy, wo, wi, pdf, type, rs);
                                     else (void)mat_sample(m, h, gx, gy, wo, wi, pdf, type);
                                     wi = normalize(wi);
                                 }
@@ -1011,8 +1011,8 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
                                     f = fown;
                                 else
                                 {
-                                    f = kLights ? mat_eval_x(S.mats, tx, m, h, wo, wi) : mat_eval(m, h, wo, wi);
-                                    float pb = kLights ? mat_pdf_x(S.mats, tx, m, h, wo, wi) : mat_pdf(m, h, wo, wi);
+                                    f = kLights ? mat_eval_x(&J.s, tx, m, h, wo, wi) : mat_eval(m, h, wo, wi);
+                                    float pb = kLights ? mat_pdf_x(&J.s, tx, m, h, wo, wi) : mat_pdf(m, h, wo, wi);
                                     pdf = alpha * pb + (guided ? (1.f - alpha) * guide_pdf(G, wi) : 0.f);
                                 }
                                 stop = !(pdf > 0.f) || sqnorm(f) == 0.f;
@@ -1023,7 +1023,7 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
                                 // gitracer.cpp:36-41), drawn again from its counter
                                 float ux, uy;
                                 nee_sample2d(J.brdf_smp, base, KS_BRDF, 0, ux, uy);
-                                f = kLights ? mat_sample_x(S.mats, tx, m, h, ux, uy, wo, wi, pdf, type, rs)
+                                f = kLights ? mat_sample_x(&J.s, tx, m, h, ux, uy, wo, wi, pdf, type, rs)
                                             : mat_sample(m, h, ux, uy, wo, wi, pdf, type);
                                 stop = sqnorm(f) == 0.f || pdf < kMinPdf;
                             }
