@@ -83,8 +83,7 @@ struct RenderWork
     DevBuf<float2> nee_b;              // MIS slots
     DevBuf<int4> nee_res;              // MIS slots
     DevBuf<uint8_t> nee_occ;           // shadow slots
-    DevBuf<float4> qc_o[2], qc_d[2], qa_o[2], qa_d[2];   // closest / any-hit queues
-    DevBuf<int> qc_own[2], qa_own[2];
+    DevBuf<uint32_t> qc[2], qa[2];     // closest / any-hit queues: the rays' owners
     DevBuf<float4> gin, rec;          // guide network inputs (2 per row), training records (per path)
     DevBuf<uint8_t> rec_state, rec_emit;   // per path: which of its training records are stored, have a weight
     DevBuf<float4> pdir;              // guided probe jobs: per path, probe ray direction and weight

@@ -118,7 +118,9 @@ struct RenderDev
     const JobDev* jobs;
     uint32_t P;        // paths in this chunk
     int Kshift;        // NEE slots per path = 1 << Kshift
-    float4 *ray_o, *ray_d, *thr, *thr_nee, *rad, *out;
+    float4 *ray_o, *ray_d;    // the path's extension ray: origin and tmin, direction and tmax; its NEE
+                              // rays share the origin
+    float4 *thr, *thr_nee, *rad, *out;
     int4* hit;
     // x: key base, y: flags | bounce << 8 | nee lights << 16 | job << 24, z/w: NEE slots with a ray in
     // flight (bit 2j: light j's shadow ray, 2j + 1: its MIS ray)
@@ -131,8 +133,7 @@ struct RenderDev
     float2* nee_b;            // per MIS slot: 1 / pdf, light
     int4* nee_res;            // per MIS slot: its ray's hit
     uint8_t* nee_occ;         // per shadow slot: 1 where the ray was blocked
-    float4 *qc_o[2], *qc_d[2], *qa_o[2], *qa_d[2];
-    int *qc_own[2], *qa_own[2];
+    uint32_t *qc[2], *qa[2];  // closest and any-hit queues: each ray's owner (queued_ray)
     uint32_t* counters;            // per launch L: closest count, any count (one 64-bit word, so a
                                    // shade wave claims both with one atomic), closest work, any work
                                    // (k_trace_queue)
@@ -194,14 +195,12 @@ __global__ void k_chunk_rays(const uint32_t* counters, int launches, unsigned lo
 __device__ __forceinline__ void init_path(const RenderDev& R, uint32_t i, f3 o, f3 d, float tmin, float tmax,
                                           uint32_t base, uint32_t job)
 {
-    R.ray_o[i] = st3(o, 0.f);
-    R.ray_d[i] = st3(d, 0.f);
+    R.ray_o[i] = st3(o, tmin);
+    R.ray_d[i] = st3(d, tmax);
     R.thr[i] = make_float4(1.f, 1.f, 1.f, 0.f);
     R.rad[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     R.meta[i] = make_uint4(base, F_EXT | (job << 24), 0u, 0u);
-    R.qc_o[0][i] = st3(o, tmin);
-    R.qc_d[0][i] = st3(d, tmax);
-    R.qc_own[0][i] = (int)((Q_EXT << 29) | i);
+    R.qc[0][i] = (Q_EXT << 29) | i;
     if (R.rec)
     {
         R.rec_state[i] = 0;
@@ -341,6 +340,22 @@ __device__ __forceinline__ size_t nee_half(const RenderDev& R, uint32_t idx)
     return nee_at(R, (idx & ((1u << R.Kshift) - 1u)) >> 1, idx >> R.Kshift);
 }
 
+// The ray of a queue entry, read from its path's state: its origin and tmin into a, its direction and
+// tmax into b. The queues hold owners only. An entry's origin, direction and owner written together
+// cost the shade kernel 36 B per ray, for shadow rays also a second read of the direction, where
+// the state holds all of it already; a wave's entries stay within the 64 paths of one shading wave,
+// so the reads here fall on the same few lines (with whole rays in the queues / owners only: Cornell
+// 256^2 1004 / 926 us, a batch of 16 scenes 9.52 / 9.10 ms, 1080p frame over 3M triangles 199.6 /
+// 196.7 ms, 4096 probes 6.83 / 6.61 ms).
+__device__ __forceinline__ void queued_ray(const RenderDev& R, uint32_t own, float4& a, float4& b)
+{
+    const uint32_t kind = own >> 29, idx = own & ((1u << 29) - 1u);
+    const uint32_t i = kind == Q_EXT ? idx : idx >> R.Kshift;
+    a = gload(R.ray_o, i);
+    b = gload(kind == Q_EXT ? R.ray_d : R.nee_wi, kind == Q_EXT ? idx : nee_at(R, idx & ((1u << R.Kshift) - 1u), i));
+    if (kind == Q_NEE_CLOSEST) b.w = 10000000.f;   // .w is the sample's MIS weight
+}
+
 __device__ __forceinline__ uint32_t path_of(const RenderDev& R, uint32_t kind, uint32_t idx)
 {
     return kind == Q_EXT ? idx : (idx >> R.Kshift);
@@ -436,9 +451,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_queue(RenderDev R, int L, int 
         }
         const uint32_t count = R.counters[4 * L + pass];
         uint32_t* work = &R.counters[4 * L + 2 + pass];
-        const float4* qo = pass == 0 ? R.qc_o[buf] : R.qa_o[buf];
-        const float4* qd = pass == 0 ? R.qc_d[buf] : R.qa_d[buf];
-        const int* qown = pass == 0 ? R.qc_own[buf] : R.qa_own[buf];
+        const uint32_t* qown = pass == 0 ? R.qc[buf] : R.qa[buf];
         for (;;)
         {
             uint32_t base = 0;
@@ -448,8 +461,9 @@ __global__ __launch_bounds__(kBlock) void k_trace_queue(RenderDev R, int L, int 
             uint32_t q = base + lane;
             if (q < count)
             {
-                float4 a = qo[q], b = qd[q];
-                uint32_t own = (uint32_t)qown[q];
+                uint32_t own = qown[q];
+                float4 a, b;
+                queued_ray(R, own, a, b);
                 uint32_t kind = own >> 29, idx = own & ((1u << 29) - 1u);
                 uint32_t job = R.meta[path_of(R, kind, idx)].y >> 24;
                 const SceneDev S = R.jobs[job].s;
@@ -562,9 +576,9 @@ k_trace_refill(RenderDev R, int L, int buf, int refill, uint32_t claim_rays)
                     const uint32_t q = (p / kWorkRun * kWorkParts + part) * kWorkRun + p % kWorkRun;
                     any = q >= nc;
                     const uint32_t k = any ? q - nc : q;
-                    const float4 a = gload(any ? R.qa_o[buf] : R.qc_o[buf], k);
-                    const float4 b = gload(any ? R.qa_d[buf] : R.qc_d[buf], k);
-                    own = (uint32_t)(any ? R.qa_own[buf][k] : R.qc_own[buf][k]);
+                    own = (any ? R.qa[buf] : R.qc[buf])[k];
+                    float4 a, b;
+                    queued_ray(R, own, a, b);
                     if (!kOne)
                     {
                         const uint32_t job = R.meta[path_of(R, own >> 29, own & ((1u << 29) - 1u))].y >> 24;
@@ -944,7 +958,6 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
                                 }
                             }
                             R.thr_nee[i] = st3(T, 0.f);
-                            R.ray_o[i] = st3(h.p, 0.f);
                             meta.z = (uint32_t)emit_mask;
                             meta.w = (uint32_t)(emit_mask >> 32);
                             if (emit_mask) fl |= F_NEE;
@@ -1062,7 +1075,7 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
                                     emit_ext = true;
                                     ext_d = nd;
                                     R.thr[i] = st3(T, 0.f);
-                                    R.ray_d[i] = st3(nd, 0.f);
+                                    R.ray_d[i] = st3(nd, 1000000.f);
                                     fl |= F_EXT;
                                 }
                                 else
@@ -1078,6 +1091,7 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
                     }
                 }
             }
+            if (emit_ext || emit_mask) R.ray_o[i] = st3(org, 0.01f);
             // ---- 3. finalise: clamp(radiance / numsamples, 0, MAXRADIANCE), gitracer.cpp:139 ----
             if ((fl & F_TERM) && !(fl & F_NEE))
             {
@@ -1192,9 +1206,7 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
             if (mine)
             {
                 const uint32_t cp = cbase + cofs + (uint32_t)__popcll(m & below);
-                R.qc_o[buf][cp] = st3(org, 0.01f);
-                R.qc_d[buf][cp] = st3(ext_d, 1000000.f);
-                R.qc_own[buf][cp] = (int)((Q_EXT << 29) | i);
+                R.qc[buf][cp] = (Q_EXT << 29) | i;
             }
             cofs += (uint32_t)__popcll(m);
         }
@@ -1205,21 +1217,8 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
             if (mine)
             {
                 const uint32_t ks = i << R.Kshift | (uint32_t)k;
-                float4 wd = R.nee_wi[nee_at(R, k, i)];
-                if (k & 1)
-                {
-                    const uint32_t cp = cbase + cofs + (uint32_t)__popcll(m & below);
-                    R.qc_o[buf][cp] = st3(org, 0.01f);
-                    R.qc_d[buf][cp] = st3(ld3(wd), 10000000.f);
-                    R.qc_own[buf][cp] = (int)((Q_NEE_CLOSEST << 29) | ks);
-                }
-                else
-                {
-                    const uint32_t ap = abase + aofs + (uint32_t)__popcll(m & below);
-                    R.qa_o[buf][ap] = st3(org, 0.01f);
-                    R.qa_d[buf][ap] = wd;
-                    R.qa_own[buf][ap] = (int)((Q_NEE_ANY << 29) | ks);
-                }
+                if (k & 1) R.qc[buf][cbase + cofs + (uint32_t)__popcll(m & below)] = (Q_NEE_CLOSEST << 29) | ks;
+                else R.qa[buf][abase + aofs + (uint32_t)__popcll(m & below)] = (Q_NEE_ANY << 29) | ks;
             }
             if (k & 1) cofs += (uint32_t)__popcll(m);
             else aofs += (uint32_t)__popcll(m);
@@ -1450,12 +1449,8 @@ static bsh_status ensure_work(RenderWork& w, size_t P, int K, int nlmax)
     size_t qc = P * (size_t)(1 + nlmax), qa = P * (size_t)std::max(nlmax, 1);
     for (int k = 0; k < 2; ++k)
     {
-        BSH_HIP(w.qc_o[k].alloc(qc));
-        BSH_HIP(w.qc_d[k].alloc(qc));
-        BSH_HIP(w.qc_own[k].alloc(qc));
-        BSH_HIP(w.qa_o[k].alloc(qa));
-        BSH_HIP(w.qa_d[k].alloc(qa));
-        BSH_HIP(w.qa_own[k].alloc(qa));
+        BSH_HIP(w.qc[k].alloc(qc));
+        BSH_HIP(w.qa[k].alloc(qa));
     }
     BSH_HIP(w.stats.alloc(kStatAll));
     return BSH_OK;
@@ -1977,8 +1972,8 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
         R.nee_occ = lw.nee_occ.p;
         for (int k = 0; k < 2; ++k)
         {
-            R.qc_o[k] = lw.qc_o[k].p; R.qc_d[k] = lw.qc_d[k].p; R.qc_own[k] = lw.qc_own[k].p;
-            R.qa_o[k] = lw.qa_o[k].p; R.qa_d[k] = lw.qa_d[k].p; R.qa_own[k] = lw.qa_own[k].p;
+            R.qc[k] = lw.qc[k].p;
+            R.qa[k] = lw.qa[k].p;
         }
         R.counters = lw.counters.p;
         R.alive_n = lw.counters.p + alive_off;
