@@ -251,7 +251,9 @@ __device__ __forceinline__ f3 probe_dir(uint32_t base, int j, int g)
     float z = 1.f - 2.f * u;
     float r = sqrtf(fmaxf(0.f, 1.f - z * z));
     float phi = 2.f * kPi * v;
-    return mk(r * cosf(phi), r * sinf(phi), z);
+    float sinphi, cosphi;
+    sin_cos(phi, sinphi, cosphi);
+    return mk(r * cosphi, r * sinphi, z);
 }
 
 // Network inputs of the probes [u0, u0+nu) of a guided probe job, rows row0.. : the probe

@@ -100,8 +100,9 @@ __device__ __forceinline__ f3 other_light_sample(const SceneDev& s, const LightD
         dist2d_sample(s.env, ux, uy, u, v, dpdf);
         float theta = v * kPi;
         float phi = u * 2.f * kPi;
-        float costheta = cosf(theta), sintheta = sinf(theta);
-        float sinphi = sinf(phi), cosphi = cosf(phi);
+        float sintheta, costheta, sinphi, cosphi;
+        sin_cos(theta, sintheta, costheta);
+        sin_cos(phi, sinphi, cosphi);
         d = 100000000.f * normalize(mk(sintheta * cosphi, costheta, sintheta * sinphi));
         pdf = sintheta == 0.f ? 0.f : dpdf / (2.f * kPi * kPi * sintheta);
     }
