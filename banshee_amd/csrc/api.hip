@@ -129,11 +129,14 @@ bsh_status bsh_context_create(int device, bsh_context** out)
     std::string arch = prop.gcnArchName;
     if (arch.rfind("gfx950", 0) != 0)
         return fail(BSH_ERR_NO_DEVICE, "bsh_context_create: device is " + arch + ", this build targets gfx950");
+    int clock_khz = 0;
+    BSH_HIP(hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, device));
     bsh_status sv = env_scratch_init(device);
     if (sv != BSH_OK) return sv;
     bsh_context* c = new bsh_context();
     c->device = device;
     c->num_cus = prop.multiProcessorCount;
+    c->clock_khz = std::max(1, clock_khz);
     c->lds_per_cu = prop.maxSharedMemoryPerMultiProcessor;
     *out = c;
     return BSH_OK;

@@ -198,11 +198,14 @@ constexpr int kFwdTiles = 2;
 // v0..v6) -> the network's outputs. Weights and biases are staged in LDS once per block; each
 // wave runs kFwdTiles 16-row tiles at a time with all activations in registers. kHalf: write only the kGUsed outputs the mixture uses, in FP16 (the wavefront's
 // form), else all kGOut in FP32. seg (when set): rows come in segments of kGuideSeg of which
-// the first seg[s] are live; tile groups past a segment's rows are skipped.
+// the first seg[s] are live; tile groups past a segment's rows are skipped. stamp (when set) receives
+// the time the kernel started.
 template <bool kHalf>
 __global__ __launch_bounds__(64 * kFwdWaves) void k_guide_forward(GuideNet g, const float4* in, int stride,
-                                                                 uint32_t nrows, const uint32_t* seg, void* outp)
+                                                                 uint32_t nrows, const uint32_t* seg, void* outp,
+                                                                 unsigned long long* stamp)
 {
+    const ClockStamp clock(stride);
     constexpr int kGroup = 16 * kFwdTiles;
     static_assert(kGuideSeg % kGroup == 0, "tile groups must not straddle segments");
     __shared__ u4v img[kImgUnits];
@@ -283,6 +286,7 @@ __global__ __launch_bounds__(64 * kFwdWaves) void k_guide_forward(GuideNet g, co
             }
         }
     }
+    clock.store(stamp);
 }
 
 constexpr float kMaxRecordWeight = 256.f;
@@ -1015,19 +1019,19 @@ bsh_status guide_forward(bsh_guide* g, const float4* in, int stride, uint32_t n,
     uint32_t groups = (n + 16 * kFwdTiles - 1) / (16 * kFwdTiles);
     uint32_t blocks = std::min<uint32_t>((groups + kFwdWaves - 1) / kFwdWaves, (uint32_t)g->ctx->num_cus * 3);
     hipLaunchKernelGGL((k_guide_forward<false>), dim3(blocks), dim3(64 * kFwdWaves), 0, st, g->net(), in,
-                       stride, n, (const uint32_t*)nullptr, (void*)out);
+                       stride, n, (const uint32_t*)nullptr, (void*)out, (unsigned long long*)nullptr);
     BSH_HIP(hipGetLastError());
     return BSH_OK;
 }
 
 bsh_status guide_forward_rows(bsh_guide* g, const float4* in, const uint32_t* seg_counts, uint32_t rows,
-                              _Float16* out, hipStream_t st)
+                              _Float16* out, hipStream_t st, unsigned long long* stamp)
 {
     if (rows == 0) return BSH_OK;
     uint32_t groups = (rows + 16 * kFwdTiles - 1) / (16 * kFwdTiles);
     uint32_t blocks = std::min<uint32_t>((groups + kFwdWaves - 1) / kFwdWaves, (uint32_t)g->ctx->num_cus * 3);
     hipLaunchKernelGGL((k_guide_forward<true>), dim3(blocks), dim3(64 * kFwdWaves), 0, st, g->net(), in, 2,
-                       rows, seg_counts, (void*)out);
+                       rows, seg_counts, (void*)out, stamp);
     BSH_HIP(hipGetLastError());
     return BSH_OK;
 }

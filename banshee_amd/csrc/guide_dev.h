@@ -138,4 +138,23 @@ __device__ __forceinline__ f3 guide_sample(const Lobes& L, const T* o, float u0,
     return normalize(mu * w + t1 * (s * __builtin_amdgcn_cosf(u2)) + t2 * (s * __builtin_amdgcn_sinf(u2)));
 }
 
+// A kernel's time stamp: the device clock at its start, that is when the kernel before it on the stream
+// had finished (the first workgroup of a grid is dispatched first). Neither reading it nor storing it
+// may look like a write to memory ahead of the kernel's uniform loads, which could not be scalar ones
+// then (k_shade's per-block read of its live-path count, a vector load behind other blocks' atomics on the
+// same line, made the kernel 2.4 times as long): the clock is read by an instruction without side
+// effects, kept in its place by the launch argument that passes through it, and stored at the end.
+struct ClockStamp
+{
+    unsigned long long t;
+    __device__ __forceinline__ explicit ClockStamp(int& arg)
+    {
+        asm("s_memrealtime %0\n\ts_waitcnt lgkmcnt(0)" : "=s"(t), "+s"(arg));
+    }
+    __device__ __forceinline__ void store(unsigned long long* p) const
+    {
+        if (p && blockIdx.x == 0 && threadIdx.x == 0) *p = t;
+    }
+};
+
 }  // namespace bsh

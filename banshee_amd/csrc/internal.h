@@ -93,7 +93,8 @@ struct RenderWork
     DevBuf<uint32_t> rec_count;       // records written so far (running over the chunks)
     DevBuf<uint32_t> rec_blk, rec_off; // per block of paths: records, output offset
     DevBuf<uint32_t> alive[2];     // paths still live after a shade, listed for the next bounce
-    DevBuf<uint32_t> counters;     // per launch: count, work, (pad) x 4; then the live-path counts
+    DevBuf<uint32_t> counters;     // per launch: count, work, (pad) x 4; then the live-path counts, the
+                                   // trace launches' work counters and the kernels' time stamps
     DevBuf<unsigned long long> stats;  // closest, any
     DevBuf<uint32_t> stk_ovf;          // deep traversal-stack entries of the trace kernel
 };
@@ -144,7 +145,7 @@ bsh_status guide_forward(bsh_guide* g, const float4* in, int stride, uint32_t n,
 // FP16. Tiles past a segment's count are skipped.
 constexpr int kGuideSeg = 256;
 bsh_status guide_forward_rows(bsh_guide* g, const float4* in, const uint32_t* seg_counts, uint32_t rows,
-                              _Float16* out, hipStream_t st);
+                              _Float16* out, hipStream_t st, unsigned long long* stamp = nullptr);
 float guide_bsdf_fraction(const bsh_guide* g);
 int guide_bounces(const bsh_guide* g);
 
@@ -159,6 +160,8 @@ struct bsh_context
     size_t lds_per_cu = 0;
     std::mutex mu;                 // serialises work on the shared buffers below
     bsh::RenderWork work;
+    int clock_khz = 0;             // rate of the device clock that kernels stamp (wall_clock64)
+    unsigned long long* stats_host = nullptr;   // pinned: a run's statistics, copied behind its last kernel
     // further wavefront lanes: a run of several chunks deals them round-robin over the lanes,
     // each extra lane with its own buffers and stream, so one chunk's kernels fill another's
     // trace drain (measured: two lanes 7.7 % on a 1080p frame; a third added nothing there
@@ -182,6 +185,7 @@ struct bsh_context
     ~bsh_context()
     {
         drop_graph();
+        if (stats_host) (void)hipHostFree(stats_host);
         if (graph_stream) (void)hipStreamDestroy(graph_stream);
         for (hipStream_t s : lane_stream)
             if (s) (void)hipStreamDestroy(s);

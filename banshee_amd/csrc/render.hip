@@ -83,7 +83,8 @@ constexpr int kShadeWavesLights = 3;
 // bounce launch b: closest rays, any-hit rays, and in counting mode node visits and triangle tests
 // of the closest and of the any-hit rays (kLaunchStat counters each).
 constexpr int kStatRows = 4, kRowParts = 64, kRowStride = 16, kStatTotal = kStatRows + kRowParts * kRowStride;
-constexpr int kMaxLaunches = 256, kLaunchStat = 6, kStatAll = kStatTotal + kMaxLaunches * kLaunchStat;
+constexpr int kMaxLaunches = 256, kLaunchStat = 7, kStatTicks = kStatTotal + kMaxLaunches * kLaunchStat,
+              kStatAll = kStatTicks + 2;
 static_assert(kMaxLaunches > 250, "a job's depth is at most 250, so a chunk has at most 251 launches");
 // Idle lanes of a wave that trigger a refill in k_trace_refill (when the tuning leaves it 0).
 // Measured on the 3M-triangle terrain at 1080p: 8 lanes 733 Mrays/s, 16 1058, 32 1314,
@@ -138,6 +139,8 @@ struct RenderDev
                                    // shade wave claims both with one atomic), closest work, any work
                                    // (k_trace_queue)
     uint32_t* work;                // per launch L: kWorkParts work counters, kWorkStride apart (k_trace_refill)
+    unsigned long long* stamp;     // per launch L: the clock at the start of its trace, guide input, inference
+                                   // and shade kernels (0: no such kernel)
     uint32_t* alive[2];            // live paths: shade b reads list b & 1, writes list (b + 1) & 1
     uint32_t* alive_n;             // per bounce: length of its live-path list (b >= 1)
     unsigned long long* stats;     // closest, any, node visits, triangle tests, then kRowParts guided-row partials
@@ -173,22 +176,47 @@ __global__ void k_set_count(uint32_t* counters, unsigned long long* stats, uint3
     if (threadIdx.x == 0) counters[0] = P;
 }
 
-// After a chunk: its closest and any-hit ray totals, from every launch's queue counts (added
-// atomically: the chunks of two lanes may finish at the same time).
-__global__ void k_chunk_rays(const uint32_t* counters, int launches, unsigned long long* stats)
+// After a chunk: its closest and any-hit ray totals, from every launch's queue counts, and the launches'
+// durations from the clock stamps (added atomically: the chunks of two lanes may finish at the same
+// time). A launch lasts until the next kernel of its stream starts. Events around the launches, which
+// the stamps replace, left the GPU idle for 25 us per bounce: a Cornell 256^2 frame of 6 launches 930 us with them, 803
+// without; mapped materials 2170 / 2035; a guided 1024^2 pass 6.49 / 6.31 ms; 4096 probes 6.65 / 6.36.
+constexpr int kStampTrace = 0, kStampInputs = 1, kStampInfer = 2, kStampShade = 3, kStamps = 4;
+__device__ __forceinline__ unsigned long long ticks(unsigned long long from, unsigned long long to)
 {
+    return to > from ? to - from : 0ull;
+}
+__global__ __launch_bounds__(64) void k_chunk_rays(const uint32_t* counters, const unsigned long long* stamp,
+                                                   int launches, unsigned long long* stats)
+{
+    const unsigned long long now = wall_clock64();
+    unsigned long long c = 0, a = 0, shade = 0, infer = 0;
+    for (int L = threadIdx.x; L < launches; L += 64)
+    {
+        const unsigned long long nc = counters[4 * L + 0], na = counters[4 * L + 1];
+        const unsigned long long* s = stamp + kStamps * L;
+        unsigned long long* ls = stats + kStatTotal + kLaunchStat * L;
+        atomicAdd(&ls[0], nc);
+        atomicAdd(&ls[1], na);
+        atomicAdd(&ls[6], ticks(s[kStampTrace], s[kStampInputs] ? s[kStampInputs] : s[kStampShade]));
+        c += nc;
+        a += na;
+        shade += ticks(s[kStampShade], L + 1 < launches ? s[kStamps + kStampTrace] : now);
+        if (s[kStampInfer]) infer += ticks(s[kStampInfer], s[kStampShade]);
+    }
+    for (int m = 1; m < 64; m <<= 1)
+    {
+        c += __shfl_xor(c, m);
+        a += __shfl_xor(a, m);
+        shade += __shfl_xor(shade, m);
+        infer += __shfl_xor(infer, m);
+    }
     if (threadIdx.x == 0)
     {
-        unsigned long long c = 0, a = 0;
-        for (int L = 0; L < launches; ++L)
-        {
-            c += counters[4 * L + 0];
-            a += counters[4 * L + 1];
-            atomicAdd(&stats[kStatTotal + kLaunchStat * L + 0], (unsigned long long)counters[4 * L + 0]);
-            atomicAdd(&stats[kStatTotal + kLaunchStat * L + 1], (unsigned long long)counters[4 * L + 1]);
-        }
         atomicAdd(&stats[0], c);
         atomicAdd(&stats[1], a);
+        atomicAdd(&stats[kStatTicks], shade);
+        atomicAdd(&stats[kStatTicks + 1], infer);
     }
 }
 
@@ -371,6 +399,7 @@ __device__ __forceinline__ uint32_t path_of(const RenderDev& R, uint32_t kind, u
 // the threads walk the live-path list the shade of this bounce will walk, not all paths.
 __global__ __launch_bounds__(kBlock) void k_guide_inputs(RenderDev R, int b)
 {
+    const ClockStamp clock(b);
     __shared__ uint32_t wsum[kBlock / 64];
     const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
     uint32_t i = t;
@@ -420,6 +449,7 @@ __global__ __launch_bounds__(kBlock) void k_guide_inputs(RenderDev R, int b)
         // lines (one shared counter serialises the blocks' atomics)
         if (total) atomicAdd(&R.stats[kStatRows + kRowStride * (blockIdx.x % kRowParts)], (unsigned long long)total);
     }
+    clock.store(R.stamp + kStamps * b + kStampInputs);
     if (!have) return;
     int row = -1;
     if (want)
@@ -434,6 +464,7 @@ __global__ __launch_bounds__(kBlock) void k_guide_inputs(RenderDev R, int b)
 template <bool kCount>
 __global__ __launch_bounds__(kBlock) void k_trace_queue(RenderDev R, int L, int buf)
 {
+    const ClockStamp clock(L);
     __shared__ uint32_t stk[kTraceLds * kBlock];
     const int lane = threadIdx.x & 63;
     uint32_t* my = stk + threadIdx.x;
@@ -504,6 +535,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_queue(RenderDev R, int L, int 
         atomicAdd(&R.stats[2], (unsigned long long)vis_nodes);
         atomicAdd(&R.stats[3], (unsigned long long)vis_tris);
     }
+    clock.store(R.stamp + kStamps * L + kStampTrace);
 }
 
 // The overflow slots of a trace thread's stack: entries past kTraceLds, [entry][trace thread].
@@ -531,6 +563,7 @@ template <bool kCount, bool kQ, bool kOne>
 __global__ __launch_bounds__(kBlock, kOne && !kCount ? kTraceResidentBlocks : kTraceResidentMulti) void
 k_trace_refill(RenderDev R, int L, int buf, int refill, uint32_t claim_rays)
 {
+    const ClockStamp clock(L);
     __shared__ __align__(16) uint32_t stk[kTraceLds * kBlock];
     const int lane = threadIdx.x & 63;
     const QueueOvf ovf{R.stk_ovf};
@@ -633,6 +666,7 @@ k_trace_refill(RenderDev R, int L, int buf, int refill, uint32_t claim_rays)
         atomicAdd(&R.stats[2], (unsigned long long)(vis_nodes + vis_nodes_any));
         atomicAdd(&R.stats[3], (unsigned long long)(vis_tris + vis_tris_any));
     }
+    clock.store(R.stamp + kStamps * L + kStampTrace);
 }
 
 // Inclusive prefix sum over the 64 lanes of a wave.
@@ -657,6 +691,7 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
 template <bool kFull, bool kOne, bool kLights = false>
 __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPerSimd) void k_shade(RenderDev R, int b, int Lout)
 {
+    const ClockStamp clock(b);
     // Bounce 0 shades every path of the chunk; a later bounce only the paths the previous
     // shade left live, in the order it listed them (its wave order, so neighbouring paths
     // stay together). A wave then holds live paths only, instead of the survivors scattered
@@ -1226,6 +1261,7 @@ __global__ __launch_bounds__(kBlock, kLights ? kShadeWavesLights : kShadeWavesPe
             else aofs += (uint32_t)__popcll(m);
         }
     }
+    clock.store(R.stamp + kStamps * b + kStampShade);
 }
 
 // ---- training records: each chunk's records are compacted in (path, vertex) order ----
@@ -1458,25 +1494,6 @@ static bsh_status ensure_work(RenderWork& w, size_t P, int K, int nlmax)
     return BSH_OK;
 }
 
-// HIP events around every trace and shade launch on the launch stream, read once at the end.
-struct LaunchTimer
-{
-    std::vector<hipEvent_t> evs;
-    std::vector<int> bounce;   // the bounce (launch index within its chunk) of every pass, in order
-    size_t ei = 0;
-    bsh_status init(size_t pairs)
-    {
-        evs.resize(5 * pairs + 2);
-        for (auto& e : evs) BSH_HIP(hipEventCreate(&e));
-        return BSH_OK;
-    }
-    hipEvent_t next() { return evs[ei++]; }
-    ~LaunchTimer()
-    {
-        for (auto& e : evs) (void)hipEventDestroy(e);
-    }
-};
-
 #define BSH_TRY(x)                   \
     do                               \
     {                                \
@@ -1540,8 +1557,6 @@ static void launch_refill(bool one, int blocks, hipStream_t st, const RenderDev&
                            claim);
 }
 
-// Enqueues every kernel of a batch on `st`. With T == nullptr no events are recorded
-// (the form captured into a hipGraph).
 // Orders further streams after a first one (fork) and the first after all of them (join).
 struct ForkJoin
 {
@@ -1585,8 +1600,7 @@ struct Lane
 
 // Enqueues every chunk of the run; chunk k goes to lane k mod nlanes.
 static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, const std::vector<Chunk>& chunks,
-                                const std::vector<JobDev>& hjobs, bool count, const bsh_tuning& tune, LaunchTimer* T,
-                                GuideRun* gr)
+                                const std::vector<JobDev>& hjobs, bool count, const bsh_tuning& tune, GuideRun* gr)
 {
     const int max_blocks = c->num_cus * std::max(1, tune.trace_blocks_per_cu);
     const int refill = tune.refill_lanes == 0 ? kDefaultRefill : tune.refill_lanes;
@@ -1655,11 +1669,6 @@ static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, c
         dim3 pg = grid_for(ch.P);
         for (int b = 0; b <= ch.depth; ++b)
         {
-            if (T)
-            {
-                BSH_HIP(hipEventRecord(T->next(), st));
-                T->bounce.push_back(b);
-            }
             if (wide)
             {
                 const bool one = R.nodes1 != nullptr;
@@ -1677,20 +1686,18 @@ static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, c
                 hipLaunchKernelGGL(k_trace_queue<true>, dim3(trace_blocks), dim3(kBlock), 0, st, R, b, b & 1);
             else
                 hipLaunchKernelGGL(k_trace_queue<false>, dim3(trace_blocks), dim3(kBlock), 0, st, R, b, b & 1);
-            if (T) BSH_HIP(hipEventRecord(T->next(), st));
             // no inference at the chunk's last bounce: no job of it samples a continuation there
             const bool infer = gr && gr->guide && b + 1 < ch.depth && (gr->bounces == 0 || b < gr->bounces);
             if (infer)
             {
                 hipLaunchKernelGGL(k_guide_inputs, pg, dim3(kBlock), 0, st, R, b);
             }
-            if (T) BSH_HIP(hipEventRecord(T->next(), st));
             if (infer)
             {
-                bsh_status gs = guide_forward_rows(gr->guide, R.gin, w.gseg.p, pg.x * kBlock, w.gout.p, st);
+                bsh_status gs = guide_forward_rows(gr->guide, R.gin, w.gseg.p, pg.x * kBlock, w.gout.p, st,
+                                                   R.stamp + kStamps * b + kStampInfer);
                 if (gs != BSH_OK) return gs;
             }
-            if (T) BSH_HIP(hipEventRecord(T->next(), st));
             const int lo = b + 1 <= ch.depth ? b + 1 : b;
             if (lights && one) hipLaunchKernelGGL((k_shade<true, true, true>), pg, dim3(kBlock), 0, st, R, b, lo);
             else if (lights) hipLaunchKernelGGL((k_shade<true, false, true>), pg, dim3(kBlock), 0, st, R, b, lo);
@@ -1698,9 +1705,9 @@ static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, c
             else if (full) hipLaunchKernelGGL((k_shade<true, false>), pg, dim3(kBlock), 0, st, R, b, lo);
             else if (one) hipLaunchKernelGGL((k_shade<false, true>), pg, dim3(kBlock), 0, st, R, b, lo);
             else hipLaunchKernelGGL((k_shade<false, false>), pg, dim3(kBlock), 0, st, R, b, lo);
-            if (T) BSH_HIP(hipEventRecord(T->next(), st));
         }
-        hipLaunchKernelGGL(k_chunk_rays, dim3(1), dim3(64), 0, st, (const uint32_t*)w.counters.p, launches, R.stats);
+        hipLaunchKernelGGL(k_chunk_rays, dim3(1), dim3(64), 0, st, (const uint32_t*)w.counters.p,
+                           (const unsigned long long*)R.stamp, launches, R.stats);
         if (R.rec_out)
         {
             hipLaunchKernelGGL(k_rec_count, pg, dim3(kBlock), 0, st, R, w.rec_blk.p);
@@ -1935,6 +1942,8 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     const size_t alive_off = ((size_t)4 * (maxdepth + 1) + 63) / 64 * 64;
     // (then, from a further 256-B boundary, the trace launches' work counters)
     const size_t work_off = (alive_off + maxdepth + 2 + 63) / 64 * 64;
+    // (and from another, the time stamps)
+    const size_t stamp_off = work_off + (size_t)(maxdepth + 1) * kWorkParts * kWorkStride;
     const size_t trace_threads = std::max<size_t>((size_t)c->num_cus * std::max(1, tune.trace_blocks_per_cu), kWorkParts) * kBlock;
     BSH_HIP(c->jobs.alloc(hjobs.size()));
     BSH_HIP(hipMemcpyAsync(c->jobs.p, hjobs.data(), hjobs.size() * sizeof(JobDev), hipMemcpyHostToDevice, st));
@@ -1944,7 +1953,7 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     // every lane's buffers and device view (the statistics are lane 0's, shared)
     auto setup_lane = [&](RenderWork& lw, RenderDev& R) -> bsh_status {
         BSH_TRY(ensure_work(lw, P, K, nlmax));
-        BSH_HIP(lw.counters.alloc(work_off + (size_t)(maxdepth + 1) * kWorkParts * kWorkStride));
+        BSH_HIP(lw.counters.alloc(stamp_off + (size_t)(maxdepth + 1) * kStamps * 2));
         if (guided)
         {
             const size_t Pb = (P + kBlock - 1) / kBlock * kBlock;   // rows live in whole segments
@@ -1980,6 +1989,7 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
         R.counters = lw.counters.p;
         R.alive_n = lw.counters.p + alive_off;
         R.work = lw.counters.p + work_off;
+        R.stamp = reinterpret_cast<unsigned long long*>(lw.counters.p + stamp_off);
         R.alive[0] = lw.alive[0].p;
         R.alive[1] = lw.alive[1].p;
         R.stats = w.stats.p;
@@ -2021,6 +2031,16 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     bsh_render_stats& S = c->stats;
     S = bsh_render_stats{};
     std::vector<double> launch_ms(maxdepth + 1, 0.0);
+    // the statistics and, of a recording run, the number of records: copied behind the run's kernels
+    // into pinned memory, with one wait
+    if (!c->stats_host) BSH_HIP(hipHostMalloc((void**)&c->stats_host, (kStatAll + 1) * sizeof(unsigned long long)));
+    unsigned long long* st2 = c->stats_host;
+    auto fetch_stats = [&]() -> bsh_status {
+        BSH_HIP(hipMemcpyAsync(st2, w.stats.p, kStatAll * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
+        if (record) BSH_HIP(hipMemcpyAsync(st2 + kStatAll, w.rec_count.p, 4, hipMemcpyDeviceToHost, st));
+        BSH_HIP(hipStreamSynchronize(st));
+        return BSH_OK;
+    };
     if (use_graph)
     {
         // Capture the whole batch (every chunk's raygen, bounces, accumulation) as one graph
@@ -2071,7 +2091,7 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
                 gl[0].st = cs;
                 ForkJoin fj;
                 if (nlanes > 1) rc = fj.fork(cs, c->lane_stream, nlanes - 1);
-                if (rc == BSH_OK) rc = enqueue_batch(c, gl, nlanes, chunks, hjobs, count, tune, nullptr, gr);
+                if (rc == BSH_OK) rc = enqueue_batch(c, gl, nlanes, chunks, hjobs, count, tune, gr);
                 if (rc == BSH_OK && nlanes > 1) rc = fj.join(cs, c->lane_stream, nlanes - 1);
                 hipError_t e2 = hipStreamEndCapture(cs, &graph);
                 if (rc == BSH_OK && e2 != hipSuccess) rc = hip_fail(e2, "hipStreamEndCapture");
@@ -2119,45 +2139,47 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
         (void)hipEventDestroy(e1);
         S.graph_replayed = replay ? 1u : 0u;
         if (rc != BSH_OK) return rc;
+        BSH_TRY(fetch_stats());
         S.trace_launches = S.shade_launches = (uint32_t)pairs;
     }
     else
     {
-        LaunchTimer T;
-        BSH_TRY(T.init(pairs));
-        BSH_HIP(hipEventRecord(T.next(), st));
+        struct Span
+        {
+            hipEvent_t e[2] = {};
+            ~Span()
+            {
+                for (hipEvent_t k : e)
+                    if (k) (void)hipEventDestroy(k);
+            }
+        } run;
+        for (hipEvent_t& e : run.e) BSH_HIP(hipEventCreate(&e));
+        BSH_HIP(hipEventRecord(run.e[0], st));
         // the second lane starts after everything before it on `st` (job table, cleared
         // statistics) and `st` continues after both lanes
         ForkJoin fj;
         if (nlanes > 1) BSH_TRY(fj.fork(st, c->lane_stream, nlanes - 1));
-        BSH_TRY(enqueue_batch(c, lanes, nlanes, chunks, hjobs, count, tune, &T, gr));
+        BSH_TRY(enqueue_batch(c, lanes, nlanes, chunks, hjobs, count, tune, gr));
         if (nlanes > 1) BSH_TRY(fj.join(st, c->lane_stream, nlanes - 1));
-        BSH_HIP(hipEventRecord(T.next(), st));
-        BSH_HIP(hipEventSynchronize(T.evs[T.ei - 1]));
-        // per pass: before trace, after trace, after the guide inputs, after inference, after shade
-        for (size_t k = 1; k + 4 < T.ei; k += 5)
-        {
-            float a = 0.f, g = 0.f, b = 0.f;
-            BSH_HIP(hipEventElapsedTime(&a, T.evs[k], T.evs[k + 1]));
-            BSH_HIP(hipEventElapsedTime(&g, T.evs[k + 2], T.evs[k + 3]));
-            BSH_HIP(hipEventElapsedTime(&b, T.evs[k + 3], T.evs[k + 4]));
-            S.trace_ms += a;
-            S.shade_ms += b;
-            launch_ms[T.bounce[(k - 1) / 5]] += a;
-            S.trace_launches++;
-            S.shade_launches++;
-            if (guided && g > 0.f)
-            {
-                S.guide_ms += g;
-                S.guide_launches++;
-            }
-        }
+        BSH_HIP(hipEventRecord(run.e[1], st));
+        BSH_TRY(fetch_stats());
         float tot = 0.f;
-        BSH_HIP(hipEventElapsedTime(&tot, T.evs[0], T.evs[T.ei - 1]));
+        BSH_HIP(hipEventElapsedTime(&tot, run.e[0], run.e[1]));
         S.total_ms = tot;
+        const double ms = 1.0 / c->clock_khz;   // of a clock tick
+        for (int b = 0; b <= maxdepth; ++b)
+        {
+            launch_ms[b] = (double)st2[kStatTotal + kLaunchStat * b + 6] * ms;
+            S.trace_ms += launch_ms[b];
+        }
+        S.shade_ms = (double)st2[kStatTicks] * ms;
+        S.trace_launches = S.shade_launches = (uint32_t)pairs;
+        if (guided)
+        {
+            S.guide_ms = (double)st2[kStatTicks + 1] * ms;
+            S.guide_launches = (uint32_t)pairs;   // every pass, as inference is part of a pass
+        }
     }
-    std::vector<unsigned long long> st2(kStatAll);
-    BSH_HIP(hipMemcpy(st2.data(), w.stats.p, kStatAll * sizeof(unsigned long long), hipMemcpyDeviceToHost));
     c->launch_stats.assign(maxdepth + 1, bsh_launch_stats{});
     for (int b = 0; b <= maxdepth; ++b)
     {
@@ -2181,7 +2203,7 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     if (record)
     {
         uint32_t nrec = 0;
-        BSH_HIP(hipMemcpy(&nrec, w.rec_count.p, 4, hipMemcpyDeviceToHost));
+        std::memcpy(&nrec, st2 + kStatAll, 4);
         gr->written = std::min<size_t>(nrec, gr->cap);
     }
     return BSH_OK;

@@ -181,7 +181,10 @@ typedef struct
     uint64_t rays_closest, rays_any;   /* BVH queries issued (Intersectable::Intersect x2) */
     uint64_t camera_samples;
     uint64_t node_visits, tri_tests;   /* totals over all queries, BSH_RENDER_COUNT only */
-    double trace_ms, shade_ms, total_ms; /* summed HIP-event durations */
+    double trace_ms, shade_ms, total_ms; /* the trace and the shade launches' durations summed (0 in graph
+                                            mode), from clock stamps at the kernels' starts: a launch
+                                            lasts until its stream's next kernel starts; the whole run
+                                            between HIP events */
     uint32_t trace_launches, shade_launches;
     uint32_t guide_launches;           /* guide network inference launches (guided render or bake) */
     uint64_t guide_rows;               /* path vertices run through the guide network */
@@ -442,7 +445,7 @@ typedef struct
     uint64_t rays_closest, rays_any;
     uint64_t nodes_closest, tris_closest;   /* node visits and triangle tests, BSH_RENDER_COUNT only */
     uint64_t nodes_any, tris_any;
-    double trace_ms;                        /* summed HIP-event durations of these launches (0 in graph mode) */
+    double trace_ms;                        /* summed durations of these launches (0 in graph mode) */
 } bsh_launch_stats;
 /* Copies min(cap, launches) entries to out and the number of launches of the last run to *n. */
 bsh_status bsh_context_launch_stats(const bsh_context* ctx, bsh_launch_stats* out, size_t cap, size_t* n);
