@@ -87,8 +87,10 @@ constexpr int kMaxLaunches = 256, kLaunchStat = 7, kStatTicks = kStatTotal + kMa
               kStatAll = kStatTicks + 2;
 static_assert(kMaxLaunches > 250, "a job's depth is at most 250, so a chunk has at most 251 launches");
 // Idle lanes of a wave that trigger a refill in k_trace_refill (when the tuning leaves it 0).
-// Measured on the 3M-triangle terrain at 1080p: 8 lanes 733 Mrays/s, 16 1058, 32 1314,
-// 48 1381, 56 1393, 64 1353; whole 64-ray batches per wave (k_trace_queue) 1065.
+// Refilling few lanes costs the whole wave an atomic and two dependent loads; waiting for more leaves
+// lanes idle. At 8 / 16 / 32 / 40 / 48 / 56 / 60 idle lanes: 1080p 64-sample frame over 3M triangles
+// 225 / 209 / 204 / 197 / 194 / 193 / 195 ms; batch of 16 scenes 11.0 / 10.1 / 9.5 / 9.3 / 9.06 / 9.00 /
+// 9.01 ms; 4096 probes 6.53 / 6.31 / 6.33 / 6.33 / 6.28 / 6.34 / 6.49 ms.
 constexpr int kDefaultRefill = 56;
 // Work counters of a k_trace_refill launch, each on a cache line of its own; the queue is dealt to
 // them in runs of kWorkRun entries. Returning atomics on one line are served about 6 ns apart, so

@@ -463,12 +463,12 @@ def ray_classes(ls, s_node, s_tri) -> dict:
 
 def isolated_launches(ctx, scene, classes, seed) -> dict:
     """One untimed frame of the workload on one wavefront lane at the two-lane default's per-lane
-    grid (3 trace workgroups per CU), so no trace launch shares the GPU with another lane: per
-    launch class, the summed HIP-event durations on the launch stream and the algorithmic bytes
+    grid (4 trace workgroups per CU), so no trace launch shares the GPU with another lane: per
+    launch class, the summed durations from device clock stamps and the algorithmic bytes
     of the rays it traced (rays x that class's B_ray)."""
     old = ctx.tuning()
     try:
-        ctx.set_tuning(0, 3, 0, 0, 0, 1)
+        ctx.set_tuning(0, 4, 0, 0, 0, 1)
         scene.render(W, H, GRID, DEPTH, seed, download=False)
         ctx.sync()
         ls = ctx.launch_stats()
@@ -639,7 +639,7 @@ def main():
     dt = time.perf_counter() - t1
 
     value = rays / dt / 1e6
-    # the dominant kernel's own launch time: the isolated frame's HIP events (no second lane)
+    # the dominant kernel's own launch time: the isolated frame's clock stamps (no second lane)
     avg_launch_s = iso["trace_ms"] / 1e3 / iso["launches"]
     bytes_per_launch = iso["bytes"] / iso["launches"]
     achieved = bytes_per_launch / avg_launch_s / 1e9
@@ -678,8 +678,8 @@ def main():
                      "traffic_source": "profiles/k_trace_refill_terrain3M_pmc.md (FETCH_SIZE x2.0 + WRITE_SIZE x1.0)",
                      "kernel": "k_trace_refill" if int(info["width"]) == 4 and args.refill_lanes != -1 else "k_trace_queue",
                      "avg_launch_ms": round(avg_launch_s * 1e3, 4),
-                     "launch_timing": "HIP events on the launch stream, in an untimed frame of the workload on one "
-                                      "lane at the default per-lane grid (3 workgroups/CU), so no launch overlaps "
+                     "launch_timing": "device clock stamps at the kernels' starts, in an untimed frame of the workload on one "
+                                      "lane at the default per-lane grid (4 workgroups/CU), so no launch overlaps "
                                       "another lane's kernels",
                      "avg_launch_ms_two_lanes": round(trace_ms / trace_launches, 4),
                      "bytes_per_ray": round(b_mix, 1), "anchored_to_steps_gbs": round(anchored, 1),
