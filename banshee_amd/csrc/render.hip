@@ -43,6 +43,7 @@
 #include "sh_dev.h"
 #include "guide_dev.h"
 #include "trace_core.h"
+#include "wave_sizes.h"
 
 namespace bsh {
 
@@ -1474,7 +1475,7 @@ __global__ __launch_bounds__(kBlock) void k_project_sh(RenderDev R, uint32_t job
 // ---------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------
-static bsh_status ensure_work(RenderWork& w, size_t P, int K, int nlmax)
+static bsh_status ensure_work(RenderWork& w, size_t P, int Kshift)
 {
     BSH_HIP(w.ray_o.alloc(P));
     BSH_HIP(w.ray_d.alloc(P));
@@ -1486,13 +1487,13 @@ static bsh_status ensure_work(RenderWork& w, size_t P, int K, int nlmax)
     BSH_HIP(w.meta.alloc(P));
     BSH_HIP(w.alive[0].alloc(P));
     BSH_HIP(w.alive[1].alloc(P));
-    size_t slots = P * (size_t)K;
+    const size_t slots = P << Kshift;
     BSH_HIP(w.nee_a.alloc(slots));
     BSH_HIP(w.nee_wi.alloc(slots));
     BSH_HIP(w.nee_b.alloc(slots / 2));
     BSH_HIP(w.nee_res.alloc(slots / 2));
     BSH_HIP(w.nee_occ.alloc(slots / 2));
-    size_t qc = P * (size_t)(1 + nlmax), qa = P * (size_t)std::max(nlmax, 1);
+    const size_t qc = P * closest_rays_per_path(Kshift), qa = P * any_rays_per_path(Kshift);
     for (int k = 0; k < 2; ++k)
     {
         BSH_HIP(w.qc[k].alloc(qc));
@@ -1626,9 +1627,8 @@ static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, c
         hipStream_t st = ln.st;
         const int launches = ch.depth + 1;
         R.P = ch.P;
-        // no more trace workgroups than the chunk's rays can use (a bounce has at most one extension
-        // ray and one ray per NEE slot and path), and one for every work counter
-        const size_t most_rays = (size_t)ch.P * (1 + ((size_t)1 << R.Kshift));
+        // no more trace workgroups than the chunk's rays can use, and one for every work counter
+        const size_t most_rays = (size_t)ch.P * (closest_rays_per_path(R.Kshift) + any_rays_per_path(R.Kshift));
         const int trace_blocks = (int)std::max<size_t>(kWorkParts, std::min<size_t>(max_blocks, (most_rays + kBlock - 1) / kBlock));
         bool full = false, lights = false, wide = refill > 0, qall = true, qany = false;
         for (const Segment& sg : ch.segs)
@@ -1886,15 +1886,13 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     bool nmaps = false;
     for (const JobDev& J : hjobs)
     {
-        // NEE slots: two per light of the bounce-0 loop, two for a picked light (four with
-        // normal maps: the second BSDF ray of a normal-mapped vertex)
+        // lights sampled at a vertex: every one in the bounce-0 loop, or one picked
         nlmax = std::max(nlmax, (J.flags & JOB_NO_QUIRKS) && J.s.nlights > kMaxNeeLights ? 1 : J.s.nlights);
         nmaps = nmaps || (J.s.nmaps && !(J.flags & JOB_NO_QUIRKS));
         maxunit = std::max<uint32_t>(maxunit, J.type == 0 ? (uint32_t)J.s_count : (uint32_t)J.N);
         samples += J.type == 0 ? (uint64_t)J.cw * J.ch * J.s_count : (uint64_t)J.nprobes * J.N;
     }
-    int Kshift = 1;
-    while ((1 << Kshift) < (nmaps ? 4 : 2) * nlmax) ++Kshift;
+    const int Kshift = nee_slot_shift(nlmax, nmaps);
     if (Kshift > 6) return fail(BSH_ERR_UNSUPPORTED, "more NEE slots per path than the 64-bit slot mask holds");
     const int K = 1 << Kshift;
     size_t pmax = std::max<size_t>((size_t)tune.paths_per_chunk, maxunit);
@@ -1955,12 +1953,12 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     const size_t trace_threads = std::max<size_t>((size_t)c->num_cus * std::max(1, tune.trace_blocks_per_cu), kWorkParts) * kBlock;
     BSH_HIP(c->jobs.alloc(hjobs.size()));
     BSH_HIP(hipMemcpyAsync(c->jobs.p, hjobs.data(), hjobs.size() * sizeof(JobDev), hipMemcpyHostToDevice, st));
-    BSH_TRY(ensure_work(c->work, P, K, nlmax));   // lane 0's buffers also hold the run's statistics
+    BSH_TRY(ensure_work(c->work, P, Kshift));   // lane 0's buffers also hold the run's statistics
     RenderWork& w = c->work;
 
     // every lane's buffers and device view (the statistics are lane 0's, shared)
     auto setup_lane = [&](RenderWork& lw, RenderDev& R) -> bsh_status {
-        BSH_TRY(ensure_work(lw, P, K, nlmax));
+        BSH_TRY(ensure_work(lw, P, Kshift));
         BSH_HIP(lw.counters.alloc(stamp_off + (size_t)(maxdepth + 1) * kStamps * 2));
         if (guided)
         {
