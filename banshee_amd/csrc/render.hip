@@ -640,7 +640,7 @@ k_trace_refill(RenderDev R, int L, int buf, int refill, uint32_t claim_rays)
         if (__ballot(active) == 0ull) break;
         if (!active) continue;
         uint32_t nv = 0, tv = 0;
-        const bool done = step4<kCount, kQ, kOne, kTraceLds, kBlock>(r, any, nodes, tris, stk, ovf, nv, tv);
+        const bool done = step4<kCount, kQ, kOne, false, kTraceLds, kBlock>(r, any, nodes, tris, stk, ovf, nv, tv);
         if (kCount)
         {
             (any ? vis_nodes_any : vis_nodes) += nv;
@@ -1607,6 +1607,10 @@ struct Lane
     hipStream_t st;
 };
 
+// Whether the refill kernel may trace the job's rays (kLeastMin): a path's first ray starts at the camera's
+// near plane or the probe job's tmin, the others at 0.01.
+static bool refill_tmin(const JobDev& J) { return (J.type == 0 ? J.cam.znear : J.tmin) >= kLeastMin; }
+
 // Enqueues every chunk of the run; chunk k goes to lane k mod nlanes.
 static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, const std::vector<Chunk>& chunks,
                                 const std::vector<JobDev>& hjobs, bool count, const bsh_tuning& tune, GuideRun* gr)
@@ -1639,7 +1643,7 @@ static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, c
             // point, directional and environment lights and the materials of rows 3-7 are compiled
             // into the kLights variants only
             lights = lights || hjobs[sg.job].s.narea != hjobs[sg.job].s.nlights || hjobs[sg.job].s.ext_mats;
-            wide = wide && hjobs[sg.job].s.width == 4;
+            wide = wide && hjobs[sg.job].s.width == 4 && refill_tmin(hjobs[sg.job]);
         }
         // the refill kernel is compiled for one 4-wide node layout; a chunk that mixes the float
         // and quantised layouts is traced by the queue kernel, which reads the layout per ray
@@ -2065,8 +2069,8 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
         put(&tune, sizeof tune);
         for (const JobDev& J : hjobs)
         {
-            const int f[13] = {J.type, J.s_count, J.N, J.cw, J.ch, J.nprobes, J.depth, J.flags,
-                               J.s.narea, J.s.nlights, J.s.ext_mats, J.s.width, J.s.qnodes};
+            const int f[14] = {J.type, J.s_count, J.N, J.cw, J.ch, J.nprobes, J.depth, J.flags,
+                               J.s.narea, J.s.nlights, J.s.ext_mats, J.s.width, J.s.qnodes, refill_tmin(J)};
             put(f, sizeof f);
         }
         for (int k = 0; k < nlanes; ++k) put(&lanes[k].R, sizeof(RenderDev));

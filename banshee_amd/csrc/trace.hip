@@ -74,7 +74,7 @@ __global__ __launch_bounds__(64, 8) void k_query4(const float4* __restrict__ nod
         }
         if (__ballot(active) == 0ull) break;
         if (!active) continue;
-        if (!step4<false, kQ, false, kQueryLds, 64>(r, kAny, nodes, tris, stk, ovf, nv, tv)) continue;
+        if (!step4<false, kQ, false, true, kQueryLds, 64>(r, kAny, nodes, tris, stk, ovf, nv, tv)) continue;
         const bool h = r.prim >= 0;
         if (kAny && occ) occ[idx] = h ? 1 : 0;
         if (hits)

@@ -14,7 +14,7 @@
 //    plane distances instead of 24 conversions, 24 fma, 3 compares and 6 selects.
 //  * Which children are hit: the sign bits of (exit - entry), replicated to bytes by v_perm, are
 //    and-ed with the node's leaf bits (the hit triangles) and turn the keys of children that are
-//    missed, leaves or empty into sentinels with one conversion and one fma each.
+//    missed, leaves or empty into sentinels with two instructions each.
 //  * The sort: a key (entry distance) and its node index are the high and low word of a double,
 //    so a compare-exchange is a v_min_f64 and a v_max_f64 instead of a compare and 4 selects.
 //  * Leaf triangles: the node's leaves hold consecutive triangles, so the next one is found by
@@ -86,14 +86,24 @@ struct LaneRay
 
 constexpr uint32_t kSelLo = 0x0c010c00u, kSelHi = 0x0c050c04u;   // bytes 0, 1 of the second / first source
 constexpr uint32_t kStackEnd = 0xffffffffu;                      // the stack's bottom entry
-// A sentinel key is at least kKeyFar; entry distances are culled above kKeyMost.
-constexpr float kKeyFar = 1.7014118e38f, kKeyMost = 1.5e38f;
+// Sentinel keys of the children that are not to be visited. With kAnyMin any tmin is allowed: the key
+// of such a child is kKeyNone, above every float's bits (+inf among them) in the order of the doubles
+// and as a float a NaN, which no comparison accepts. Without it tmin is at least kLeastMin, so
+// every entry distance is, and the sentinel is formed by an fma: at least kKeyFar + kLeastMin, above
+// kKeyMost, beyond which entry distances are culled. (With an entry distance of -1e38 or -inf the
+// fma would give a leaf's key a value to be visited, as a node, at its first triangle's index.) The
+// selecting form takes one instruction more per visit: 1080p frame 191.1 ms with the fma, 192.6
+// with the selection, 700,001 shadow rays 156.7 / 157.6 us. The wavefront, whose tmin the host
+// knows, takes the fma, the ray queries the selection.
+constexpr uint32_t kKeyNone = 0x7f900000u;
+constexpr float kKeyFar = 1.7014118e38f, kKeyMost = 1.5e38f, kLeastMin = -1e37f;
 
 typedef _Float16 th2 __attribute__((ext_vector_type(2)));
 
 // Visits `node`: the hit leaf triangles (pend) and the internal children's keys. kQ: GpuNodeQ
-// nodes, else GpuNode4. kOne: `nodes` is the same for every lane and smaller than 4 GiB.
-template <bool kQ, bool kOne>
+// nodes, else GpuNode4. kOne: `nodes` is the same for every lane and smaller than 4 GiB. kAnyMin: see
+// kKeyNone.
+template <bool kQ, bool kOne, bool kAnyMin>
 __device__ __forceinline__ void visit4(LaneRay& r, const float4* nodes, uint32_t node)
 {
     float tn[4], df[4];
@@ -172,13 +182,33 @@ __device__ __forceinline__ void visit4(LaneRay& r, const float4* nodes, uint32_t
     r.base = (uint32_t)ref[0] - 1u;
     r.full = leaf;
     r.pend = leaf & ~miss;
-    // key = entry distance + (0 for a hit internal child, else >= kKeyFar); a leaf's count is
-    // positive and an empty child's byte is 0xff
+    // key = the entry distance of a hit internal child, else a sentinel; a leaf's count is 1 to 8 and
+    // an empty or missed child's byte 0xff
     const uint32_t out = miss | cnts;
-    r.k0 = key_pair(__builtin_fmaf((float)(out & 0xffu), kKeyFar, tn[0]), (uint32_t)ref[0]);
-    r.k1 = key_pair(__builtin_fmaf((float)((out >> 8) & 0xffu), kKeyFar, tn[1]), (uint32_t)ref[1]);
-    r.k2 = key_pair(__builtin_fmaf((float)((out >> 16) & 0xffu), kKeyFar, tn[2]), (uint32_t)ref[2]);
-    r.k3 = key_pair(__builtin_fmaf((float)(out >> 24), kKeyFar, tn[3]), (uint32_t)ref[3]);
+    double key[4];
+    if (kAnyMin)
+    {
+        // as v_perm selectors those bytes pick 0xff, and 0 picks 0
+        uint32_t lut = 0xffffff00u, none = kKeyNone;
+        asm("" : "+s"(lut), "+s"(none));   // in scalar registers, not moved or combined in vector ones
+        const uint32_t skip = __builtin_amdgcn_perm(0xffffffffu, lut, out);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+        {
+            const uint32_t m = __builtin_amdgcn_perm(skip, skip, 0x01010101u * (uint32_t)c);
+            key[c] = key_pair(__uint_as_float((m & none) | (~m & __float_as_uint(tn[c]))), (uint32_t)ref[c]);
+        }
+    }
+    else
+    {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            key[c] = key_pair(__builtin_fmaf((float)((out >> (8 * c)) & 0xffu), kKeyFar, tn[c]), (uint32_t)ref[c]);
+    }
+    r.k0 = key[0];
+    r.k1 = key[1];
+    r.k2 = key[2];
+    r.k3 = key[3];
 }
 
 // The lane's stack: `top` in a register, the other entries in LDS ([entry][lane], kStride lanes),
@@ -227,7 +257,7 @@ __device__ __forceinline__ void start_ray(LaneRay& r, uint32_t* stk, float4 a, f
 // One step of an active lane: a pending leaf triangle, then, once the lane's leaves are done, its
 // internal children (culled against the closest hit, nearest first) and the next node's visit.
 // The order of box and triangle tests is traverse4's. Returns true when the ray is finished.
-template <bool kCount, bool kQ, bool kOne, int kLds, int kStride, class Ovf>
+template <bool kCount, bool kQ, bool kOne, bool kAnyMin, int kLds, int kStride, class Ovf>
 __device__ __forceinline__ bool step4(LaneRay& r, bool any, const float4* nodes, const float4* tris, uint32_t* stk,
                                       const Ovf& ovf, uint32_t& nvis, uint32_t& tvis)
 {
@@ -262,7 +292,8 @@ __device__ __forceinline__ bool step4(LaneRay& r, bool any, const float4* nodes,
         pair_sort2(r.k1, r.k3);
         pair_sort2(r.k1, r.k2);
         // the children not beyond the closest hit are the first ones of the sorted four
-        const float tc = fminf(r.tcur, kKeyMost);
+        // (entered at +inf, a child is not visited in either form)
+        const float tc = fminf(r.tcur, kAnyMin ? 3.4028235e38f : kKeyMost);
         const bool c0 = pair_key(r.k0) <= tc, c1 = pair_key(r.k1) <= tc, c2 = pair_key(r.k2) <= tc,
                    c3 = pair_key(r.k3) <= tc;
         uint32_t node = pair_id(r.k0);
@@ -308,7 +339,7 @@ __device__ __forceinline__ bool step4(LaneRay& r, bool any, const float4* nodes,
         if (!done)
         {
             if (kCount) ++nvis;
-            visit4<kQ, kOne>(r, nodes, node);
+            visit4<kQ, kOne, kAnyMin>(r, nodes, node);
         }
     }
     return done;
