@@ -29,15 +29,16 @@ bsh_status hip_fail(hipError_t e, const char* what)
     return BSH_ERR_HIP;
 }
 
-// Every launch-shape parameter a tuning may carry, checked before any work is enqueued:
-// trace workgroups per CU are bounded by the trace kernel's LDS stack; a claim must cover a
-// whole wave's idle lanes (64), or a wave's reserve would hand out entries past its claim.
+// Every launch-shape parameter a tuning may carry, checked before any work is enqueued. Trace workgroups
+// per CU: 0, the automatic grid (render.hip), which may be larger than the 1..5 a caller may ask for; a
+// claim must cover a whole wave's idle lanes (64), or a wave's reserve would hand out entries
+// past its claim.
 bsh_status validate_tuning(const bsh_tuning& t, const char* who)
 {
     const std::string w(who);
     if (t.paths_per_chunk < 0) return fail(BSH_ERR_INVALID, w + ": paths_per_chunk must be >= 0");
     if (t.trace_blocks_per_cu < 0 || t.trace_blocks_per_cu > 5)
-        return fail(BSH_ERR_INVALID, w + ": trace_blocks_per_cu must be 0..5 (LDS limit)");
+        return fail(BSH_ERR_INVALID, w + ": trace_blocks_per_cu must be 0..5");
     if (t.refill_lanes < -1 || t.refill_lanes > 64) return fail(BSH_ERR_INVALID, w + ": refill_lanes must be -1..64");
     if (t.claim_rays != 0 && (t.claim_rays < 64 || t.claim_rays > 4096))
         return fail(BSH_ERR_INVALID, w + ": claim_rays must be 0 or 64..4096");
@@ -981,19 +982,21 @@ bsh_status bsh_autotune(bsh_context* ctx, const bsh_job* jobs, size_t njobs, con
 {
     if (!ctx || (njobs && !jobs)) return fail(BSH_ERR_INVALID, "bsh_autotune: NULL argument");
     static const int32_t kPaths[] = {1 << 21, 1 << 22, 1 << 23, 1 << 24};
-    static const int32_t kBlocks[] = {2, 3, 4, 5};
+    // the automatic grid among them (it is 4 on two lanes and 8 on one, where 4 is never the fastest)
+    static const int32_t kBlocks[] = {2, 3, 5, 0};
+    const bool sweep = !blocks_per_cu || n_blocks == 0;
     if (!paths_per_chunk || n_paths == 0) { paths_per_chunk = kPaths; n_paths = 4; }
-    if (!blocks_per_cu || n_blocks == 0) { blocks_per_cu = kBlocks; n_blocks = 4; }
+    if (sweep) { blocks_per_cu = kBlocks; n_blocks = 4; }
     std::vector<JobDev> hj;
     bool count = false;
     bsh_status r = build_jobs(ctx, jobs, njobs, hj, count);
     if (r != BSH_OK) return r;
     bsh_tuning bt = ctx->tuning;
-    double bms = 1e300;
+    double bms = 1e300, bcost = 1e300;
     for (size_t a = 0; a < n_paths; ++a)
         for (size_t b = 0; b < n_blocks; ++b)
         {
-            if (blocks_per_cu[b] < 1 || blocks_per_cu[b] > 5 || paths_per_chunk[a] < 1)
+            if (blocks_per_cu[b] < (sweep ? 0 : 1) || blocks_per_cu[b] > 5 || paths_per_chunk[a] < 1)
                 return fail(BSH_ERR_INVALID, "bsh_autotune: candidate out of range");
             bsh_tuning t{paths_per_chunk[a], blocks_per_cu[b], 0, ctx->tuning.refill_lanes, ctx->tuning.claim_rays,
                           ctx->tuning.lanes};
@@ -1002,9 +1005,12 @@ bsh_status bsh_autotune(bsh_context* ctx, const bsh_job* jobs, size_t njobs, con
             std::vector<JobDev> copy = hj;
             r = run_jobs(ctx, copy, false, &t, 0, nullptr);
             if (r != BSH_OK) return r;
-            double ms = ctx->stats.total_ms;
-            if (ms < bms)
+            const double ms = ctx->stats.total_ms;
+            // single runs differ by up to 1 %, for which the automatic grid is not given up
+            const double cost = blocks_per_cu[b] == 0 ? 0.99 * ms : ms;
+            if (cost < bcost)
             {
+                bcost = cost;
                 bms = ms;
                 bt = t;
             }

@@ -451,7 +451,9 @@ typedef struct
 bsh_status bsh_context_launch_stats(const bsh_context* ctx, bsh_launch_stats* out, size_t cap, size_t* n);
 /* Autotuner: times the batch under every candidate (paths_per_chunk x trace_blocks_per_cu),
    ncand each, and stores the fastest as the context tuning (also returned in best).
-   The jobs' outputs are overwritten. NULL candidate arrays use the built-in sweep. */
+   The jobs' outputs are overwritten. NULL candidate arrays use the built-in sweep, whose
+   trace_blocks_per_cu holds 0, the automatic grid: it is kept unless another candidate is
+   more than 1 % faster. */
 bsh_status bsh_autotune(bsh_context* ctx, const bsh_job* jobs, size_t njobs, const int32_t* paths_per_chunk,
                         size_t n_paths, const int32_t* blocks_per_cu, size_t n_blocks, bsh_tuning* best,
                         double* best_ms);
