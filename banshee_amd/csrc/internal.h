@@ -138,6 +138,7 @@ struct GuideRun
     size_t cap = 0;
     size_t written = 0;
     int bounces = 0;              // guided vertices per path (0 = all)
+    uint32_t launches = 0;        // out: inference launches over path vertices
 };
 bsh_status guide_forward(bsh_guide* g, const float4* in, int stride, uint32_t n, float* out, hipStream_t st);
 // Inference for the wavefront: rows of 2-float4 inputs in segments of kGuideSeg rows, of

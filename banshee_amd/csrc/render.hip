@@ -1709,6 +1709,7 @@ static bsh_status enqueue_batch(bsh_context* c, const Lane* lanes, int nlanes, c
                 bsh_status gs = guide_forward_rows(gr->guide, R.gin, w.gseg.p, pg.x * kBlock, w.gout.p, st,
                                                    R.stamp + kStamps * b + kStampInfer);
                 if (gs != BSH_OK) return gs;
+                ++gr->launches;
             }
             const int lo = b + 1 <= ch.depth ? b + 1 : b;
             if (lights && one) hipLaunchKernelGGL((k_shade<true, true, true>), pg, dim3(kBlock), 0, st, R, b, lo);
@@ -2184,12 +2185,9 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
         }
         S.shade_ms = (double)st2[kStatTicks] * ms;
         S.trace_launches = S.shade_launches = (uint32_t)pairs;
-        if (guided)
-        {
-            S.guide_ms = (double)st2[kStatTicks + 1] * ms;
-            S.guide_launches = (uint32_t)pairs;   // every pass, as inference is part of a pass
-        }
+        if (guided) S.guide_ms = (double)st2[kStatTicks + 1] * ms;
     }
+    if (guided) S.guide_launches = gr->launches;
     c->launch_stats.assign(maxdepth + 1, bsh_launch_stats{});
     for (int b = 0; b <= maxdepth; ++b)
     {

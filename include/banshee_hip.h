@@ -186,9 +186,11 @@ typedef struct
                                             lasts until its stream's next kernel starts; the whole run
                                             between HIP events */
     uint32_t trace_launches, shade_launches;
-    uint32_t guide_launches;           /* guide network inference launches (guided render or bake) */
+    uint32_t guide_launches;           /* guide network inference launches over path vertices (guided render
+                                          or bake): per chunk, the bounces that sample a guided
+                                          continuation, at most max_depth - 1 */
     uint64_t guide_rows;               /* path vertices run through the guide network */
-    double guide_ms;                   /* summed duration of the inference launches */
+    double guide_ms;                   /* summed duration of these launches */
     uint32_t graph_replayed;           /* bsh_batch_run with use_graph: 1 when the run replayed the context's
                                           previous graph (same jobs' shapes, tuning and buffers), 0 when it
                                           captured one */
