@@ -63,11 +63,12 @@ __global__ __launch_bounds__(kShBlock) void k_env_partial(const float* __restric
     {
         const double a = (double)(phi0 + (float)phi * phistep);
         const float sp = (float)sin(a), cp = (float)cos(a);
-        const int iu = (int)floorf((float)phi / W * W);
+        // (from 2^24 columns or rows on the quotient may round up to 1, past the last texel)
+        const int iu = min((int)floorf((float)phi / W * W), W - 1);
 #pragma unroll 4
         for (int r = row0 + sub; r < row1; r += nsub)
         {
-            const int iv = (int)floorf((float)r / H * H);
+            const int iv = min((int)floorf((float)r / H * H), H - 1);
             const float* e = env + 3 * ((size_t)W * iv + iu);
             const float st = s_sin[r - row0], ct = s_cos[r - row0], w = s_w[r - row0];
             const float ex = e[0] * w, ey = e[1] * w, ez = e[2] * w;
