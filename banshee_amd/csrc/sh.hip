@@ -9,14 +9,12 @@
 #include <string>
 #include <vector>
 
+#include "env_tiles.h"
 #include "internal.h"
 #include "sh_dev.h"
 
 namespace bsh {
 
-constexpr int kShBlock = 256;
-// Blocks of the environment projection: two per CU.
-constexpr int kEnvMaxBlocks = 512;
 // The context's scratch for it (128 KB at lmax 4 and a map up to kEnvMaxBlocks x 256 columns wide,
 // and some more for maps whose rows need more blocks).
 constexpr size_t kEnvCtxFloats = (size_t)2 * kEnvMaxBlocks * 3 * kShMaxTerms;
@@ -31,9 +29,8 @@ constexpr size_t kEnvCtxFloats = (size_t)2 * kEnvMaxBlocks * 3 * kShMaxTerms;
 // coefficient and 256 cells: 2048 x 1024, lmax 2: 88 -> 13 us, and pass 2, whose one block walked
 // 8192 partial sums per coefficient, 1634 -> 4 us; the call, which also filled its angle tables on
 // the host and allocated, with 262,144 irradiances 1773 -> 33 us.
-constexpr int kShTile = 256;
 template <int LMAX>
-__global__ __launch_bounds__(kShBlock) void k_env_partial(const float* __restrict__ env, int W, int H, int cols, int rows,
+__global__ __launch_bounds__(kShBlock) void k_env_partial(const float* __restrict__ env, int W, int H, EnvTiles tiles,
                                                         float* __restrict__ partial)
 {
     constexpr int NT = (LMAX + 1) * (LMAX + 1);
@@ -45,9 +42,10 @@ __global__ __launch_bounds__(kShBlock) void k_env_partial(const float* __restric
     // cosines rounded from double
     const float thetastep = kPi / H, phistep = 2.f * kPi / W;
     const float theta0 = kPi / H / 2, phi0 = 2.f * kPi / W / 2;
-    const int nx = (W + cols - 1) / cols, bx = blockIdx.x % nx;
-    const int row0 = blockIdx.x / nx * rows, row1 = min(row0 + rows, H);
-    if (row0 + t < row1)
+    const int cols = tiles.cols;
+    const EnvTile tile = env_tile(blockIdx.x, tiles, H);
+    const int row0 = tile.row0, nrows = tile.row1 - row0;
+    if (t < nrows)
     {
         const double a = (double)(theta0 + (float)(row0 + t) * thetastep);
         s_sin[t] = (float)sin(a);
@@ -55,7 +53,7 @@ __global__ __launch_bounds__(kShBlock) void k_env_partial(const float* __restric
         s_w[t] = s_sin[t] * thetastep * phistep;
     }
     __syncthreads();
-    const int phi = bx * cols + t % cols, sub = t / cols, nsub = kShBlock / cols;
+    const int phi = tile.col0 + t % cols, sub = t / cols, nsub = kShBlock / cols;
     float c[3 * NT];
 #pragma unroll
     for (int i = 0; i < 3 * NT; ++i) c[i] = 0.f;
@@ -66,11 +64,11 @@ __global__ __launch_bounds__(kShBlock) void k_env_partial(const float* __restric
         // (from 2^24 columns or rows on the quotient may round up to 1, past the last texel)
         const int iu = min((int)floorf((float)phi / W * W), W - 1);
 #pragma unroll 4
-        for (int r = row0 + sub; r < row1; r += nsub)
+        for (int k = sub; k < nrows; k += nsub)
         {
-            const int iv = min((int)floorf((float)r / H * H), H - 1);
+            const int iv = min((int)floorf((float)(row0 + k) / H * H), H - 1);
             const float* e = env + 3 * ((size_t)W * iv + iu);
-            const float st = s_sin[r - row0], ct = s_cos[r - row0], w = s_w[r - row0];
+            const float st = s_sin[k], ct = s_cos[k], w = s_w[k];
             const float ex = e[0] * w, ey = e[1] * w, ez = e[2] * w;
             float y[NT];
             sh_poly<LMAX>(st * cp, ct, st * sp, y);
@@ -155,25 +153,6 @@ __global__ void k_diag_sh(int lmax, uint32_t n, const float* dirs, float* out)
     for (int i = 0; i < nt; ++i) out[(size_t)t * nt + i] = y[i];
 }
 
-// Tiling of a map: `cols` columns and `rows` rows per block, about two blocks per CU where the map
-// is large enough and at most kEnvMaxBlocks.
-struct EnvTiles
-{
-    int cols, rows, nx, ny;
-};
-static EnvTiles env_tiles(int W, int H)
-{
-    EnvTiles t;
-    t.cols = 1;
-    while (t.cols < W && t.cols < kShTile) t.cols *= 2;
-    t.nx = (int)(((int64_t)W + t.cols - 1) / t.cols);
-    const int sub = kShBlock / t.cols;   // rows a block reads at a time
-    const int want = std::max(1, kEnvMaxBlocks / t.nx);
-    t.rows = std::max(sub, (H + want - 1) / want);
-    t.rows = std::min(t.rows, kShBlock);   // a block's angle table
-    t.ny = (H + t.rows - 1) / t.rows;
-    return t;
-}
 static size_t env_partial_floats(int W, int H, int lmax)
 {
     const EnvTiles t = env_tiles(W, H);
@@ -199,11 +178,11 @@ static hipError_t launch_env_projection(const float* env, int W, int H, int lmax
     const dim3 g((uint32_t)(q.nx * q.ny)), b(kShBlock);
     switch (lmax)
     {
-    case 0: hipLaunchKernelGGL(k_env_partial<0>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
-    case 1: hipLaunchKernelGGL(k_env_partial<1>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
-    case 2: hipLaunchKernelGGL(k_env_partial<2>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
-    case 3: hipLaunchKernelGGL(k_env_partial<3>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
-    default: hipLaunchKernelGGL(k_env_partial<4>, g, b, 0, st, env, W, H, q.cols, q.rows, partial); break;
+    case 0: hipLaunchKernelGGL(k_env_partial<0>, g, b, 0, st, env, W, H, q, partial); break;
+    case 1: hipLaunchKernelGGL(k_env_partial<1>, g, b, 0, st, env, W, H, q, partial); break;
+    case 2: hipLaunchKernelGGL(k_env_partial<2>, g, b, 0, st, env, W, H, q, partial); break;
+    case 3: hipLaunchKernelGGL(k_env_partial<3>, g, b, 0, st, env, W, H, q, partial); break;
+    default: hipLaunchKernelGGL(k_env_partial<4>, g, b, 0, st, env, W, H, q, partial); break;
     }
     hipLaunchKernelGGL(k_env_final, dim3(3 * (lmax + 1) * (lmax + 1)), dim3(64), 0, st, (const float*)partial,
                        q.nx * q.ny, coeffs);
