@@ -67,18 +67,19 @@ static_assert(kGuideSeg == kBlock, "guide row segments are the blocks of k_guide
 // pass on one lane 8.91 / 8.49 / 8.27 / 8.16 / 8.09.
 constexpr int kTraceBlocksOneLane = 8;
 constexpr int kTraceBlocksPerLane = 4;
-// k_trace_refill's launch bounds. One scene: 64 VGPRs, 8 workgroups per CU, without spills (80
-// VGPRs and 6 workgroups: frame 247 ms against 235, before the work counters were split). Several
+// k_trace_refill's launch bounds. One scene: 64 VGPRs, 8 workgroups per CU, without spills for the
+// quantised nodes and 12 B of them per lane for the float nodes (80 VGPRs and 6 workgroups: frame
+// 247 ms against 235, before the work counters were split). Several
 // scenes: 72 VGPRs, since at 64 the per-lane array pointers spill (batch of 16 scenes 13.0 ms
 // against 10.85; 80 VGPRs 10.87).
 constexpr int kTraceResidentBlocks = 8, kTraceResidentMulti = 7;
-// The shade kernel is held to 128 VGPRs: 4 waves per SIMD (at 129 it would run 3). Holding the
-// plain variant to 5 or 6 waves (96 or 80 VGPRs, 24 or 50 of them spilled) made the 1080p
-// terrain frame 1.1 and 1.5 % slower.
+// The shade kernel is held to 128 VGPRs: 4 waves per SIMD (at 129 it would run 3); a lane spills 20 B
+// with one job, 28 B with several. Holding the plain variant to 5 or 6 waves (96 or 80 VGPRs, 24
+// or 50 of them spilled), when it did not spill at 128, made the 1080p terrain frame 1.1 and 1.5 % slower.
 constexpr int kShadeWavesPerSimd = 4;
-// The kLights variants keep 168 VGPRs (3 waves per SIMD), of which a lane spills 48 B around the
-// material calls: a 637x361 9-sample frame of mapped materials 2525 us with 4 waves (208 B), 2340
-// with 3, 2690 with 2 (no spills).
+// The kLights variants keep 168 VGPRs (3 waves per SIMD); a lane has 76 B of scratch around the
+// material calls with one job, 108 B with several. A 637x361 9-sample frame of mapped materials,
+// when that was 48 B: 2525 us with 4 waves (208 B), 2340 with 3, 2690 with 2 (no spills).
 constexpr int kShadeWavesLights = 3;
 // Statistics buffer: 4 counters, then the guided-row partials, kRowStride apart (128 B), then per
 // bounce launch b: closest rays, any-hit rays, and in counting mode node visits and triangle tests
@@ -1902,8 +1903,9 @@ bsh_status run_jobs(bsh_context* c, std::vector<JobDev>& hjobs, bool count, cons
     const int K = 1 << Kshift;
     size_t pmax = std::max<size_t>((size_t)tune.paths_per_chunk, maxunit);
     if (pmax * (size_t)K >= ((size_t)1 << 29)) pmax = (((size_t)1 << 29) - 1) / K;
-    // the NEE slot buffers (64 B per slot) hold pmax x K slots: at most 2^27 (8 GiB) per lane, so a
-    // scene with many lights runs fewer paths per chunk
+    // the NEE slot buffers hold pmax x K slots of 44.5 B (32 B for every slot, 24 B more for a MIS slot
+    // and 1 B for a shadow slot): at most 2^27 (5.6 GiB) per lane, so a scene with many lights runs
+    // fewer paths per chunk
     if (pmax * (size_t)K > ((size_t)1 << 27)) pmax = std::max<size_t>(((size_t)1 << 27) / K, maxunit);
     if (pmax < maxunit) return fail(BSH_ERR_UNSUPPORTED, "unit larger than the NEE slot space");
     std::vector<Chunk> chunks = plan_chunks(hjobs, pmax);

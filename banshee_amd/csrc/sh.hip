@@ -15,8 +15,8 @@
 
 namespace bsh {
 
-// The context's scratch for it (128 KB at lmax 4 and a map up to kEnvMaxBlocks x 256 columns wide,
-// and some more for maps whose rows need more blocks).
+// The context's scratch for it: twice the 150 KB that kEnvMaxBlocks blocks' sums take at lmax 4, since
+// maps of many columns or rows need more blocks.
 constexpr size_t kEnvCtxFloats = (size_t)2 * kEnvMaxBlocks * 3 * kShMaxTerms;
 
 // Environment projection: c_i = sum over the map's cells of e Y_i(w) sin(theta) (pi / H) (2 pi / W).

@@ -327,7 +327,9 @@ bsh_status bsh_scene_info(const bsh_scene* s, uint64_t* nodes, uint64_t* tris, u
 
 /* ---------------- ray queries (Intersectable, accelerator/intersectable.h:41-49) ---------------- */
 /* Intersectable::Intersect(ray const&, Hit&) -> Bvh::Intersect closest hit (bvh.cpp:499-573).
-   Device pointers. */
+   Where several triangles are hit at exactly the same t, which of them is reported depends on the
+   tree (a node's leaves are tested before its internal children, those nearest first, by node
+   index where they are entered at the same distance); all calls on one scene agree. Device pointers. */
 bsh_status bsh_intersect_closest(bsh_scene* s, const bsh_ray* rays, size_t n, bsh_hit* hits, void* stream);
 /* Intersectable::Intersect(ray const&) -> Bvh::Intersect any hit (bvh.cpp:575-647).
    occluded[i] = 1 if any triangle has tmin < t <= tmax. Device pointers. */
